@@ -127,14 +127,54 @@ __device__ __forceinline__ int pi32(int i) { return ((i >> 2) & 1) * 16 + (i >> 
 // queue sizes) are each cut into W parts by key blocks, W minimising ceil(rem W / slots) / W: the parts of an item
 // run on different blocks, each writes O / l and lse of its keys, and merge_kernel combines them afterwards
 // (log-sum-exp weights). ws[3] holds the number of split items, the split table their (segment, tile, head, W).
-__device__ inline int plan_upper_bound(const int* a, int n, int x) {
-  int lo = 0, hi = n;
-  while (lo < hi) {
-    int mid = (lo + hi) >> 1;
-    if (a[mid] <= x) lo = mid + 1;
-    else hi = mid;
+//
+// Bound by latency: nothing here is more than a few KB, so the time is the launch, one round of dependent loads, the
+// barriers and one round of stores. Hence: every load of a segment goes out at once and its fields wait in LDS
+// (kPlanSmall segments); up to that many segments are ranked by counting instead of a bitonic network; a scan is
+// shuffles within a wavefront and one barrier; the divisions of the split rule and of the queues run in lanes side by
+// side; and every item finds its own place in its queue, so that no thread writes a whole segment-head.
+// Kernel time before (1024 threads, scans of ten barrier pairs each, one thread per unit's items, events read back) and
+// now: scene layer of 4 segments x 2 heads 23.9 -> 8.4 us, 12 packed sequences x 16 heads 9.6 -> 6.5, three scenes x 16
+// heads with value runs 12.5 -> 9.0, two dense sequences x 16 heads 7.2 -> 5.8 (about 2 us of each is the launch).
+constexpr int kPlanSmall = 512;       // segments whose fields are kept in LDS and ranked by counting
+constexpr int kPlanSmallThreads = 256;
+
+// a segment's fields, as its item records need them
+struct PlanSeg {
+  int q_beg, lq, q_src0, k_beg;   // first query, query count, first source row, first key
+  int lk, row, vlead, klead;      // key count (as given), first in-place token row, in-place values and keys
+};
+
+// exclusive scan over the block's threads of N values side by side: x[i] becomes the sum of the earlier threads' x[i],
+// total[i] the sum over all of them. wsum: N x 16 words of LDS that no other scan uses (one barrier).
+template <int N>
+__device__ __forceinline__ void plan_scan(int (&x)[N], int (&total)[N], int* wsum) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, waves = blockDim.x >> 6;
+  int incl[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) incl[i] = x[i];
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1)
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const int y = __shfl_up(incl[i], o, 64);
+      if (lane >= o) incl[i] += y;
+    }
+  if (lane == 63)
+#pragma unroll
+    for (int i = 0; i < N; ++i) wsum[i * 16 + w] = incl[i];
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    int before = 0, all = 0;
+    for (int k = 0; k < waves; ++k) {
+      const int y = wsum[i * 16 + k];
+      if (k < w) before += y;
+      all += y;
+    }
+    x[i] = before + incl[i] - x[i];
+    total[i] = all;
   }
-  return lo;
 }
 
 __global__ __launch_bounds__(kPlanThreads) void plan_kernel(const int32_t* cu_q, const int32_t* cu_k,
@@ -146,150 +186,193 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(const int32_t* cu_q,
                                                             int max_items, int slots, int split_keys, int parts_cap,
                                                             VRunArgs vra, int32_t* ws) {
   __shared__ unsigned long long key[kMaxPlanSeg];
-  __shared__ int off[kMaxPlanSeg + 1];
-  __shared__ int part[kPlanThreads];
+  __shared__ int off[kMaxPlanSeg + 1];          // query tiles of the sorted segments before i
+  __shared__ int s8[kQueues][kMaxPlanSeg / kQueues];
+  __shared__ int wsum[(kQueues + 1) * 16];
+  __shared__ PlanSeg cache[kPlanSmall];
   __shared__ int min_nb, split_w;
-  __shared__ int q_n[kQueues], q_s[kQueues], q_first[kQueues], q_sb[kQueues], q_tot[kQueues];
-  const int tid = threadIdx.x;
+  __shared__ int q_n[kQueues], q_s[kQueues], q_first[kQueues], q_sb[kQueues];
+  const int tid = threadIdx.x, nt = blockDim.x;
+  const bool small = n_seg <= kPlanSmall;
+  auto load_seg = [&](int s) {
+    PlanSeg x;
+    const int qa = cu_q[s], qb = cu_q[s + 1];
+    int ka = 0, kb = 0;
+    if (!k_len || !k_off) {
+      ka = cu_k[s];
+      kb = cu_k[s + 1];
+    }
+    x.q_beg = qa;
+    x.lq = qb - qa;
+    x.q_src0 = seg_q_src ? seg_q_src[s] : qa;
+    x.k_beg = k_off ? k_off[s] : ka;
+    x.lk = k_len ? k_len[s] : kb - ka;
+    x.row = v_row ? v_row[s] : 0;
+    x.vlead = v_lead ? v_lead[s] : 0;
+    x.klead = k_lead ? k_lead[s] : 0;
+    return x;
+  };
+  auto seg_of = [&](int s) { return small ? cache[s] : load_seg(s); };
+  auto key_of = [](int lk, int s) {
+    return ((unsigned long long)(0x7fffffffu - (unsigned)max(lk, 0)) << 32) | (unsigned)s;
+  };
   if (tid == 0) min_nb = 0x7fffffff;
   int n2 = 1;
-  while (n2 < n_seg) n2 <<= 1;
-  for (int i = tid; i < n2; i += kPlanThreads) {
-    if (i < n_seg) {
-      int lk = k_len ? k_len[i] : cu_k[i + 1] - cu_k[i];
-      lk = lk < 0 ? 0 : lk;
-      key[i] = ((unsigned long long)(0x7fffffffu - (unsigned)lk) << 32) | (unsigned)i;
-    } else {
-      key[i] = ~0ull;
+  if (small) {
+    for (int i = tid; i < n_seg; i += nt) {
+      const PlanSeg x = load_seg(i);
+      cache[i] = x;
+      key[i] = key_of(x.lk, i);
     }
-  }
-  __syncthreads();
-  for (int k = 2; k <= n2; k <<= 1) {
-    for (int j = k >> 1; j > 0; j >>= 1) {
-      for (int i = tid; i < n2; i += kPlanThreads) {
-        int ixj = i ^ j;
-        if (ixj > i) {
-          unsigned long long x = key[i], y = key[ixj];
-          bool up = (i & k) == 0;
-          if ((x > y) == up) {
-            key[i] = y;
-            key[ixj] = x;
+    __syncthreads();
+    unsigned long long mine[kPlanSmall / kPlanSmallThreads];
+    int rank[kPlanSmall / kPlanSmallThreads];
+#pragma unroll
+    for (int e = 0; e < kPlanSmall / kPlanSmallThreads; ++e) {
+      const int i = tid + e * nt;
+      rank[e] = -1;
+      if (i < n_seg) {
+        mine[e] = key[i];
+        int r = 0;
+        for (int j = 0; j < n_seg; ++j) r += key[j] < mine[e];   // the keys differ in their low words
+        rank[e] = r;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < kPlanSmall / kPlanSmallThreads; ++e)
+      if (rank[e] >= 0) key[rank[e]] = mine[e];
+    __syncthreads();
+  } else {
+    while (n2 < n_seg) n2 <<= 1;
+    for (int i = tid; i < n2; i += nt)
+      key[i] = i < n_seg ? key_of(k_len ? k_len[i] : cu_k[i + 1] - cu_k[i], i) : ~0ull;
+    __syncthreads();
+    for (int k = 2; k <= n2; k <<= 1) {
+      for (int j = k >> 1; j > 0; j >>= 1) {
+        for (int i = tid; i < n2; i += nt) {
+          int ixj = i ^ j;
+          if (ixj > i) {
+            unsigned long long x = key[i], y = key[ixj];
+            bool up = (i & k) == 0;
+            if ((x > y) == up) {
+              key[i] = y;
+              key[ixj] = x;
+            }
           }
         }
-      }
-      __syncthreads();
-    }
-  }
-  // items per sorted segment, exclusive scan (each thread owns a run of consecutive entries)
-  const int per = (n_seg + kPlanThreads - 1) / kPlanThreads;
-  int local = 0;
-  for (int e = 0; e < per; ++e) {
-    int i = tid * per + e;
-    if (i < n_seg) {
-      int s = (int)(key[i] & 0xffffffffu);
-      int lq = cu_q[s + 1] - cu_q[s];
-      int tiles = lq > 0 ? (lq + bq - 1) / bq : 0;
-      off[i] = tiles * H;
-      local += tiles * H;
-      if (tiles > 0) {
-        // the fewest key blocks of any item (a key-split item keeps at least one block per part)
-        int lk_min = (int)(0x7fffffffu - (unsigned)(key[i] >> 32));
-        if (k_len_head)
-          for (int h = 0; h < H; ++h) lk_min = min(lk_min, max(k_len_head[(int64_t)s * H + h], 0));
-        atomicMin(&min_nb, (lk_min + 31) / 32);
+        __syncthreads();
       }
     }
   }
-  part[tid] = local;
-  __syncthreads();
-  for (int o = 1; o < kPlanThreads; o <<= 1) {
-    int x = tid >= o ? part[tid - o] : 0;
-    __syncthreads();
-    part[tid] += x;
-    __syncthreads();
-  }
-  int run = part[tid] - local;
+  // tiles per sorted segment, exclusive scan (each thread owns a run of consecutive entries)
+  const int per = (n_seg + nt - 1) / nt;
+  int local[1] = {0}, n_tiles[1];
   for (int e = 0; e < per; ++e) {
-    int i = tid * per + e;
+    const int i = tid * per + e;
     if (i < n_seg) {
-      int c = off[i];
-      off[i] = run;
-      run += c;
+      const int s = (int)(key[i] & 0xffffffffu);
+      const int lq = small ? cache[s].lq : cu_q[s + 1] - cu_q[s];
+      const int tiles = lq > 0 ? (lq + bq - 1) / bq : 0;
+      off[i] = tiles;
+      local[0] += tiles;
+      // the fewest key blocks of any item (a key-split item keeps at least one block per part)
+      if (tiles > 0 && split_keys) atomicMin(&min_nb, ((int)(0x7fffffffu - (unsigned)(key[i] >> 32)) + 31) / 32);
     }
   }
-  if (tid == kPlanThreads - 1) off[n_seg] = part[tid];
+  if (split_keys && k_len_head) {
+    int lo = 0x7fffffff;
+    for (int x = tid; x < n_seg * H; x += nt) {
+      const int s = x / H;
+      if ((small ? cache[s].lq : cu_q[s + 1] - cu_q[s]) > 0) lo = min(lo, (max(k_len_head[x], 0) + 31) / 32);
+    }
+    if (lo != 0x7fffffff) atomicMin(&min_nb, lo);
+  }
+  plan_scan<1>(local, n_tiles, wsum);
+  {
+    int run = local[0];
+    for (int e = 0; e < per; ++e) {
+      const int i = tid * per + e;
+      if (i < n_seg) {
+        const int c = off[i];
+        off[i] = run;
+        run += c;
+      }
+    }
+  }
+  if (tid == 0) off[n_seg] = n_tiles[0];
   __syncthreads();
   // the host's bound guarantees that the items fit; if they did not, every queue stays empty and no item is written
-  const bool fits = off[n_seg] <= max_items;
-  const int total = fits ? off[n_seg] : 0;
-  // off[i] / H: query tiles of the sorted segments before i, each counted once
-  const int all_tiles = total / H;
+  const bool fits = (int64_t)n_tiles[0] * H <= max_items;
+  const int all_tiles = fits ? n_tiles[0] : 0;
+  const int total = all_tiles * H;
   auto heads_of = [&](int q) { return (H - q + kQueues - 1) / kQueues; };   // heads h < H with h % 8 == q
   // With H not a multiple of 8 (single-head views of the bounded memory: H = 1) dealing by head would leave queues
   // empty or uneven: there the unit u = i H + h (sorted segment i, head h) goes to queue u mod 8, so that every
-  // queue holds whole segment-heads in LPT order. Its place in the queue is the sum of the tiles of the units before
-  // it there: rows of 8 consecutive units, per-queue exclusive scans over the rows.
+  // queue holds whole segment-heads in LPT order. Segment i' puts H / 8 units into every queue and one more into the
+  // queues q with (q - i' H) mod 8 < H mod 8, which depends on i' mod 8 only: the tiles before a unit of segment i in
+  // its queue follow from the tiles of the earlier segments per residue i' mod 8 (s8, per row of 8 segments).
   const bool by_unit = H % kQueues != 0;
-  const int n_units = by_unit && fits ? n_seg * H : 0;
-  const int n_rows8 = (n_units + kQueues - 1) / kQueues;
-  const int rpt = (n_rows8 + kPlanThreads - 1) / kPlanThreads;   // rows of units per thread
-  const int r_lo = min(tid * rpt, n_rows8), r_hi = min(r_lo + rpt, n_rows8);
-  auto unit_tiles = [&](int u) {
-    const int i = u / H;
-    return (off[i + 1] - off[i]) / H;
-  };
-  int uexcl[kQueues];
+  const int hq = H / kQueues, hr = H % kQueues;
+  auto one_more = [&](int q, int r) { return ((q - r * hr) & (kQueues - 1)) < hr; };
+  int res_total[kQueues];
   if (by_unit) {
-    int loc[kQueues];
+    int c[kQueues];
 #pragma unroll
-    for (int q = 0; q < kQueues; ++q) loc[q] = 0;
-    for (int r = r_lo; r < r_hi; ++r)
-#pragma unroll
-      for (int q = 0; q < kQueues; ++q)
-        if (r * kQueues + q < n_units) loc[q] += unit_tiles(r * kQueues + q);
-#pragma unroll
-    for (int q = 0; q < kQueues; ++q) {
-      part[tid] = loc[q];
-      __syncthreads();
-      for (int o = 1; o < kPlanThreads; o <<= 1) {
-        const int x = tid >= o ? part[tid - o] : 0;
-        __syncthreads();
-        part[tid] += x;
-        __syncthreads();
-      }
-      uexcl[q] = part[tid] - loc[q];
-      if (tid == kPlanThreads - 1) q_tot[q] = part[tid];
-      __syncthreads();
+    for (int r = 0; r < kQueues; ++r) {
+      const int i = tid * kQueues + r;
+      c[r] = fits && i < n_seg ? off[i + 1] - off[i] : 0;
     }
+    plan_scan<kQueues>(c, res_total, wsum + 16);
+    if (tid < kMaxPlanSeg / kQueues)
+#pragma unroll
+      for (int r = 0; r < kQueues; ++r) s8[r][tid] = c[r];
   }
-  if (tid == 0) {
-    int W = 1;
+  if (tid < 64) {
+    // the split rule: length of the last round in items, ceil(rem w / slots) / w, for w parts per item
     const int rem = slots > 0 ? total % slots : 0;
+    const int ww = max(tid, 1);
+    const float v = slots > 0 ? (float)((rem * ww + slots - 1) / slots) / (float)ww : 1.0f;
+    int W = 1;
     // with many rounds of items the GPU is at its power limit through the last one too, and blocks left idle at the
     // end let the busy ones clock higher: splitting pays only for a few rounds (measured: none at 12.75 rounds,
     // 7% at 3 rounds, 2.5-3x below one round)
     if (split_keys && rem > 0 && total < kSplitMaxRounds * slots) {
-      float best = 1.0f;   // length of the last round in items: ceil(rem W / slots) / W
-      for (int w = 2; w <= kMaxSplitWays && w <= min_nb && (rem + kQueues) * w <= parts_cap; ++w) {
-        const float v = (float)((rem * w + slots - 1) / slots) / (float)w;
-        if (v < best - 1e-6f) {
-          best = v;
+      float best = 1.0f;
+      for (int w = 2; w <= kMaxSplitWays; ++w) {
+        const float x = __shfl(v, w, 64);
+        if (w <= min_nb && (rem + kQueues) * w <= parts_cap && x < best - 1e-6f) {
+          best = x;
           W = w;
         }
       }
     }
+    const int q = tid & (kQueues - 1);   // every group of 8 lanes holds the 8 queues
+    int n;
+    if (by_unit) {
+      n = hq * all_tiles;
+#pragma unroll
+      for (int r = 0; r < kQueues; ++r)
+        if (one_more(q, r)) n += res_total[r];
+    } else {
+      n = all_tiles * heads_of(q);
+    }
+    const int sq = W > 1 ? min(n, (int)(((int64_t)rem * n + total - 1) / total)) : 0;
     int first = 0, sb = 0;
-    for (int q = 0; q < kQueues; ++q) {
-      const int n = by_unit ? (fits ? q_tot[q] : 0) : all_tiles * heads_of(q);
-      const int sq = W > 1 ? min(n, (int)(((int64_t)rem * n + total - 1) / total)) : 0;
+    for (int x = 0; x < kQueues; ++x) {
+      const int nx = __shfl(n, x, 64), sx = __shfl(sq, x, 64);
+      if (x < q) {
+        first += nx + sx * (W - 1);
+        sb += sx;
+      }
+    }
+    if (tid < kQueues) {
       q_n[q] = n;
       q_s[q] = sq;
       q_first[q] = first;
       q_sb[q] = sb;
-      first += n + sq * (W - 1);
-      sb += sq;
     }
-    split_w = W;
+    if (tid == 0) split_w = W;
   }
   __syncthreads();
   const int W = split_w;
@@ -301,31 +384,36 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(const int32_t* cu_q,
   }
   int32_t* tab = ws + kWsHeader + (int64_t)kItemWords * (max_items + parts_cap);
   if (blockIdx.x == 0 && tid == 0) ws[3] = W > 1 ? q_sb[kQueues - 1] + q_s[kQueues - 1] : 0;
-  // value events of every segment (block 0): the leading run's end, then each further run's whole key blocks (its
-  // start and its end), clipped as the key loop's in-place blocks are (inside the segment's whole blocks and the
-  // token rows, past the leading run and the run before); a run starting where the stream would return to the
-  // packed rows replaces that event
-  if (blockIdx.x == 0 && vra.runs) {
-    for (int s = tid; s < n_seg; s += kPlanThreads) {
+  // value events of every segment (the last block): the leading run's end, then each further run's whole key blocks
+  // (its start and its end), clipped as the key loop's in-place blocks are (inside the segment's whole blocks and the
+  // token rows, past the leading run and the run before); a run starting where the stream would return to the packed
+  // rows replaces that event, so an event is stored when the next one is known
+  if (blockIdx.x == gridDim.x - 1 && vra.runs) {
+    for (int s = tid; s < n_seg; s += nt) {
+      int runs[3 * OR_VALUE_RUNS];
+#pragma unroll
+      for (int x = 0; x < 3 * OR_VALUE_RUNS; ++x) runs[x] = vra.runs[(int64_t)s * OR_VALUE_RUNS * 3 + x];
       int4* L = vra.events + (int64_t)s * kVEvents;
-      const int lk_seg = max(k_len ? k_len[s] : cu_k[s + 1] - cu_k[s], 0);
-      const int64_t k_beg = k_off ? k_off[s] : cu_k[s];
+      const PlanSeg g = seg_of(s);
+      const int lk_seg = max(g.lk, 0);
+      const int64_t k_beg = g.k_beg;
       const int bmax = lk_seg / 32;
-      const int row = v_row ? v_row[s] : -1, lead = v_lead ? v_lead[s] : 0;
+      const int row = v_row ? g.row : -1, lead = g.vlead;
       int64_t la = row >= 0 && lead > 0 ? min((int64_t)lead, (int64_t)lk_seg) / 32 : 0;
       if (row >= 0) la = min(la, (vra.n_vtok - row) / 32);
       la = la < 0 ? 0 : la;
       int n = 0;
+      int4 last = make_int4(kNoEvent, 0, 0, 0);   // not stored yet
       auto add = [&](int blk, uint64_t at) {
-        if (n > 0 && L[n - 1].x == blk) --n;   // superseded at the same block
-        L[n++] = make_int4(blk, (int)(uint32_t)at, (int)(uint32_t)(at >> 32), 0);
+        if (last.x != kNoEvent && last.x != blk) L[n++] = last;
+        last = make_int4(blk, (int)(uint32_t)at, (int)(uint32_t)(at >> 32), 0);
       };
       auto packed_at = [&](int blk) { return vra.v + (uint64_t)((k_beg + 32 * (int64_t)blk) * vra.rsb); };
       if (la > 0) add((int)la, packed_at((int)la));
       int prev = (int)la;
+#pragma unroll
       for (int r = 0; r < OR_VALUE_RUNS; ++r) {
-        const int32_t* e = vra.runs + ((int64_t)s * OR_VALUE_RUNS + r) * 3;
-        const int x0 = e[0], cnt = e[1], t = e[2];
+        const int x0 = runs[3 * r], cnt = runs[3 * r + 1], t = runs[3 * r + 2];
         if (cnt <= 0 || x0 < 0 || t < 0) continue;
         int bs = (x0 + 31) / 32, be = (int)min((int64_t)(x0 + (int64_t)cnt) / 32, (int64_t)bmax);
         be = (int)min((int64_t)be, (vra.n_vtok - t + x0) / 32);   // token rows t + 32 B - x0 + i < n_vtok
@@ -335,26 +423,47 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(const int32_t* cu_q,
         add(be, packed_at(be));
         prev = be;
       }
+      if (last.x != kNoEvent) L[n++] = last;
       for (; n < kVEvents; ++n) L[n] = make_int4(kNoEvent, 0, 0, 0);
     }
   }
-  // the record(s) of tile t of head `head` of sorted segment i, at position pos of queue q (the last q_s[q] positions
-  // of a queue are items split into W key parts)
-  auto emit = [&](int i, int head, int t, int q, int pos) {
+  // the record(s) of item `it` in the order (sorted segment, head, tile); the last q_s[q] positions of a queue are
+  // items split into W key parts
+  for (int it = tid + blockIdx.x * nt; it < total; it += nt * gridDim.x) {
+    int lo = 0, hi = n_seg;   // the segment i with off[i] H <= it < off[i + 1] H (it has tiles)
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) >> 1;
+      if (off[mid] * H <= it) lo = mid;
+      else hi = mid - 1;
+    }
+    const int i = lo;
+    const int tiles = off[i + 1] - off[i], local_it = it - off[i] * H;
+    const int head = local_it / tiles, t = local_it - head * tiles;
+    int q, pos;   // position within queue q
+    if (by_unit) {
+      q = (i * hr + head) & (kQueues - 1);
+      const int row8 = i / kQueues;
+      pos = hq * off[i] + (head / kQueues) * tiles + t;
+#pragma unroll
+      for (int r = 0; r < kQueues; ++r)
+        if (one_more(q, r)) {
+          pos += s8[r][row8];
+          const int x = row8 * kQueues + r;
+          if (x < i) pos += off[x + 1] - off[x];
+        }
+    } else {
+      q = head % kQueues;
+      pos = off[i] * heads_of(q) + (head / kQueues) * tiles + t;
+    }
     const int s = (int)(key[i] & 0xffffffffu);
-    const int lq = cu_q[s + 1] - cu_q[s];
+    const PlanSeg g = seg_of(s);
     const int keep = q_n[q] - q_s[q];
-    const int q_beg = cu_q[s];
-    const int k_beg = k_off ? k_off[s] : cu_k[s];
-    const int lk_seg = k_len ? k_len[s] : cu_k[s + 1] - cu_k[s];
-    const int lk = k_len_head ? min(k_len_head[(int64_t)s * H + head], lk_seg) : lk_seg;   // this head's keys
-    const int q_src0 = seg_q_src ? seg_q_src[s] : q_beg;
-    const int vl = v_lead ? v_lead[s] : 0, vr = v_row ? v_row[s] : 0, kl = k_lead ? k_lead[s] : 0;
+    const int lk = k_len_head ? min(k_len_head[(int64_t)s * H + head], g.lk) : g.lk;   // this head's keys
     auto put = [&](int64_t entry, int pw, int sidx) {
       int32_t* e = ws + kWsHeader + kItemWords * entry;
-      *(int4*)e = make_int4((t << 8) | head, pw, sidx, q_beg);
-      *(int4*)(e + 4) = make_int4(lq, q_src0, k_beg, lk < 0 ? 0 : lk);
-      *(int4*)(e + 8) = make_int4(vr, vl, kl, vra.runs ? s * kVEvents : -1);
+      *(int4*)e = make_int4((t << 8) | head, pw, sidx, g.q_beg);
+      *(int4*)(e + 4) = make_int4(g.lq, g.q_src0, g.k_beg, lk < 0 ? 0 : lk);
+      *(int4*)(e + 8) = make_int4(g.row, g.vlead, g.klead, vra.runs ? s * kVEvents : -1);
     };
     if (pos < keep) {
       put(q_first[q] + pos, 0, 0);
@@ -365,27 +474,6 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(const int32_t* cu_q,
       tab[3 * sidx + 1] = (t << 8) | head;
       tab[3 * sidx + 2] = W;
     }
-  };
-  if (by_unit) {
-    for (int r = r_lo; r < r_hi; ++r)
-#pragma unroll
-      for (int q = 0; q < kQueues; ++q) {
-        const int u = r * kQueues + q;
-        if (u >= n_units) break;
-        const int tiles = unit_tiles(u);
-        if ((int)(u % gridDim.x) == (int)blockIdx.x)
-          for (int t = 0; t < tiles; ++t) emit(u / H, u % H, t, q, uexcl[q] + t);
-        uexcl[q] += tiles;
-      }
-    return;
-  }
-  for (int it = tid + blockIdx.x * kPlanThreads; it < total; it += kPlanThreads * gridDim.x) {
-    const int i = plan_upper_bound(off, n_seg + 1, it) - 1;
-    const int tiles = (off[i + 1] - off[i]) / H;
-    const int local_it = it - off[i];
-    const int head = local_it / tiles, t = local_it - head * tiles;
-    const int q = head % kQueues;
-    emit(i, head, t, q, (off[i] / H) * heads_of(q) + (head / kQueues) * tiles + t);   // position within queue q
   }
 }
 
@@ -1310,8 +1398,9 @@ int launch_varlen(const or_varlen_args& x, void* wsp, int64_t cap, hipStream_t s
   // the planner needs key counts only: k_len when given, else the cu_k differences. It writes every word of the
   // workspace the other kernels read (queue headers, item list, split table) before they run.
   // the item records are written by up to 8 blocks (each derives the same queues), about 1024 items per block
+  const int plan_threads = x.n_seg <= kPlanSmall ? kPlanSmallThreads : kPlanThreads;
   const int plan_blocks = (int)std::min<int64_t>(8, std::max<int64_t>(1, (max_items + 1023) / 1024));
-  hipLaunchKernelGGL(plan_kernel, dim3(plan_blocks), dim3(kPlanThreads), 0, st, x.cu_q, x.cu_k,
+  hipLaunchKernelGGL(plan_kernel, dim3(plan_blocks), dim3(plan_threads), 0, st, x.cu_q, x.cu_k,
                      x.k_len ? x.k_off : nullptr,
                      x.k_len, x.seg_q_src, x.v_tok ? x.v_lead : nullptr, x.v_tok || x.k_tok ? x.v_row : nullptr,
                      x.k_tok ? x.k_lead : nullptr, x.k_len_head,
