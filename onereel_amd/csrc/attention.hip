@@ -15,6 +15,8 @@
 //   blocks ahead; rows past a segment's end read as zeros.
 // - head_dim 128: attn8_kernel, 64 queries per wavefront (one wavefront per SIMD), O in AGPRs, key loop in generated
 //   asm. head_dim 64: attn4_kernel, 32 queries per wavefront, two wavefronts per SIMD.
+// - head_dim 128 with at most 256 keys per segment: attn_short_kernel, keys and values of a segment-head in LDS for the
+//   whole item, no planner and no queues.
 // - Softmax in base 2, p = 2^(c (s - m)) with c = scale * log2(e), and a running max m raised only when needed.
 // - Optional RoPE on the Q load (table row per packed query), with the rounding of diffusers apply_rotary_emb.
 #include <math.h>
@@ -1221,6 +1223,292 @@ __global__ __launch_bounds__(kThreads) void merge_kernel(AttnArgs a, const int32
   }
 }
 
+// ------------------------------------------------------------------------------------------------------------------
+// Short key ranges (head_dim 128, at most kShortKeys keys per segment: cross-attention to a sentence). Such a call reads
+// q and writes o (2 x 256 B per query and head) and does only 4 x 128 x Lk FLOP for them: below ~400 keys it is bound by
+// HBM, and the item machinery of attn8_kernel (a ring fill, an epilogue and a claim per 256 queries, for 4 key blocks
+// of matrix work) is what it spends its time on. Here a block loads a segment-head's K and V into LDS once (LDS DMA,
+// swizzled as in the ring kernels) and its wavefronts stream the queries past them, 32 at a time and independently of
+// each other: no barrier after the load, the next 32 queries in flight while this tile computes, the scores of 128 keys
+// in registers at once (one max, no running rescale up to 128 keys), the output through LDS so that a row's 128-byte
+// lines are stored whole. Two wavefronts per SIMD: NB = 4 (128 keys, 80 KB of LDS) two blocks of 4 wavefronts per CU,
+// NB = 8 (256 keys, 160 KB) one block of 8.
+// A block finds its item (query range of a segment, head) from cu_q by itself, so there is no planner launch; items of
+// the same rows and consecutive heads run side by side, so that whole q / o rows stream through.
+// Measured against the ring kernel with its planner (with lse): 16 x 13 200 queries x 24 heads, 64 keys 1000 -> 550 us
+// (4.7 TB/s; a device copy reaches 5.5), 128 keys 1090 -> 570, 200 keys 1240 -> 795, 256 keys 1285 -> 865; 880 + 1100 +
+// 880 queries x 24 heads, 128 keys 54 (planner, attention and merge kernels) -> 14. Between 128 and 256 keys the matrix and vector work of a
+// CU (one block of 8 wavefronts) is as long as the stream. 256 to 2048 queries per item measured alike.
+// Past 128 keys the scores of a tile don't fit the registers beside O: chunks of up to 3 blocks, whose running max moves
+// only when a probability would pass 2^kShortRaise (chunks of 4 spilled: 1450 us at 256 keys).
+constexpr int kShortKeys = 256;
+constexpr int kShortSegs = 256;   // a block finds its segment 64 at a time
+
+constexpr float kShortRaise = 16.0f;   // log2 of the largest probability kept relative to an older max
+
+// LDS byte addresses of this lane's operands in slot 0: K step k (8), V^T rows of 32 dims db (4). Every read is one of
+// them plus a constant that fits the instruction's offset (formed from one base per read they took 60 registers).
+struct ShortLds {
+  uint32_t k[8], v[4];
+};
+
+struct ShortTile {
+  bf16x8 q[8];
+  f32x16 acc[4];
+  float m, l;
+};
+
+// one chunk of N key blocks (the segment's last block among them when `valid` < 16: this lane half's keys there) of a
+// 32-query tile: scores, softmax against the chunks before (FIRST: none), PV. qnext: this lane's next query, loaded
+// into t.q once the scores are done with it (nullptr: not the tile's last chunk).
+template <int N, bool FIRST>
+__device__ __forceinline__ void short_chunk(ShortTile& t, const ShortLds& ad, const int b0, int valid, float c,
+                                            const uint16_t* qnext) {
+  constexpr int SLOT = kBKB * 128 * 2;   // bytes
+  typedef __attribute__((address_space(3))) char lds_char;
+  typedef __attribute__((address_space(3))) const bf16x8 lds_bf16x8;
+  typedef __attribute__((address_space(3))) bf16x4 lds_bf16x4;
+  f32x16 s[N];
+#pragma unroll
+  for (int b = 0; b < N; ++b) {
+    const f32x16 zero = {};
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+      s[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(lds_bf16x8*)((lds_char*)(uintptr_t)ad.k[k] + (b0 + b) * SLOT),
+                                                     t.q[k], k == 0 ? zero : s[b], 0, 0, 0);
+    if (!FIRST || N == 4) __builtin_amdgcn_sched_barrier(0);
+  }
+  if (qnext)
+#pragma unroll
+    for (int k = 0; k < 8; ++k) t.q[k] = as_bf16x8(*(const u32x4*)(qnext + 16 * k));
+  if (valid < 16)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) s[N - 1][r] = r < valid ? s[N - 1][r] : -__builtin_inff();
+  float mx = max16(s[0]);
+#pragma unroll
+  for (int b = 1; b < N; ++b) mx = fmaxf(mx, max16(s[b]));
+  mx = pair_max(mx);
+  if constexpr (FIRST) {
+    t.m = mx;
+    t.l = 0.0f;
+  } else if (__any(!((mx - t.m) * c <= kShortRaise))) {
+    // the running max moves only when some probability would exceed 2^kShortRaise (O and l stay relative to it)
+    const float mn = fmaxf(t.m, mx);
+    const float alpha = __builtin_amdgcn_exp2f((t.m - mn) * c);
+#pragma unroll
+    for (int db = 0; db < 4; ++db)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) t.acc[db][r] *= alpha;
+    t.l *= alpha;
+    t.m = mn;
+  }
+  const float mc = t.m * c;
+#pragma unroll
+  for (int b = 0; b < N; ++b) {
+    bf16x8 p[2];
+    t.l += exp_pack(s[b], c, mc, p);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int half = 0; half < 2; ++half)
+#pragma unroll
+      for (int db = 0; db < 4; ++db) {
+        const f32x16 zero = {};
+        lds_char* at = (lds_char*)(uintptr_t)ad.v[db] + (b0 + b) * SLOT + 8 * half * 256;
+        const u32x2 lo = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)at));
+        const u32x2 hi = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)(at + 4 * 256)));
+        t.acc[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(u32x4{lo[0], lo[1], hi[0], hi[1]}), p[half],
+                                                            FIRST && b == 0 && half == 0 ? zero : t.acc[db], 0, 0, 0);
+      }
+  }
+}
+
+// a block's item: `rows` queries from packed query q0 on, of a segment with Lk keys
+struct ShortItem {
+  int head, q0, rows, Lk;
+};
+
+__device__ __forceinline__ const uint16_t* short_q(const AttnArgs& a, const ShortItem& x, int t, int l32, int h) {
+  // this lane's query of tile t (past the item: its last row, not used)
+  return a.q + (int64_t)(x.q0 + min(32 * t + l32, x.rows - 1)) * a.qs + x.head * 128 + 8 * h;
+}
+
+// normalise and store a tile: two halves of 64 dims through this wavefront's LDS rows `st` (16-byte chunk c of row i at
+// c ^ (i mod 8)), then 8 lanes per row store a 128-byte line
+__device__ __forceinline__ void short_store(const AttnArgs& a, const ShortItem& x, const ShortTile& t, int tt, int lane,
+                                            uint16_t* st) {
+  const int l32 = lane & 31, h = lane >> 5;
+  const float ltot = pair_sum(t.l), inv = x.Lk > 0 ? 1.0f / ltot : 0.0f;
+  if (a.lse && h == 0 && 32 * tt + l32 < x.rows)
+    a.lse[(int64_t)x.head * a.sum_q + x.q0 + 32 * tt + l32] =
+        x.Lk > 0 ? t.m * a.scale + logf(ltot) : -__builtin_inff();
+#pragma unroll
+  for (int dh = 0; dh < 2; ++dh) {
+#pragma unroll
+    for (int db = 0; db < 2; ++db)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const f32x16& o = t.acc[2 * dh + db];
+        *(uint2*)(st + l32 * 64 + (((4 * db + g) ^ (l32 & 7)) * 8 + 4 * h)) =
+            make_uint2(pack2(o[4 * g] * inv, o[4 * g + 1] * inv), pack2(o[4 * g + 2] * inv, o[4 * g + 3] * inv));
+      }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the wavefront's own rows, written by its other lanes
+#pragma unroll
+    for (int n = 0; n < 4; ++n) {
+      const int i = 8 * n + (lane >> 3), ch = lane & 7;
+      const u32x4 y = *(const u32x4*)(st + i * 64 + ((ch ^ (i & 7)) * 8));
+      if (32 * tt + i < x.rows)
+        __builtin_nontemporal_store(
+            y, (u32x4*)(a.o + (int64_t)(x.q0 + 32 * tt + i) * a.os + x.head * 128 + 64 * dh + 8 * ch));
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // read before the next half is written
+  }
+}
+
+// the item's tiles w, w + NW, ... of this wavefront against NBC key blocks in LDS
+template <int NBC, int NW>
+__device__ __forceinline__ void short_tiles(const AttnArgs& a, const ShortItem& x, const ShortLds& ad, int w, int lane,
+                                            uint16_t* st) {
+  // up to 4 blocks in one chunk; more in chunks of up to 3 (their scores beside the live accumulators)
+  constexpr int N0 = NBC <= 4 ? NBC : 3, N1 = NBC <= 4 ? 0 : NBC <= 6 ? NBC - 3 : NBC - 5, N2 = NBC - N0 - N1;
+  const int l32 = lane & 31, h = lane >> 5;
+  const int valid = x.Lk - (NBC - 1) * kBKB - 16 * h;
+  ShortTile t;
+  const uint16_t* qp = short_q(a, x, w, l32, h);
+#pragma unroll
+  for (int k = 0; k < 8; ++k) t.q[k] = as_bf16x8(*(const u32x4*)(qp + 16 * k));
+  for (int tt = w; 32 * tt < x.rows; tt += NW) {
+    const uint16_t* qn = short_q(a, x, tt + NW, l32, h);
+    if constexpr (N1 == 0) {
+      short_chunk<N0, true>(t, ad, 0, valid, a.c, qn);
+    } else {
+      short_chunk<N0, true>(t, ad, 0, 16, a.c, nullptr);
+      if constexpr (N2 == 0) {
+        short_chunk<N1, false>(t, ad, N0, valid, a.c, qn);
+      } else {
+        short_chunk<N1, false>(t, ad, N0, 16, a.c, nullptr);
+        short_chunk<N2, false>(t, ad, N0 + N1, valid, a.c, qn);
+      }
+    }
+    short_store(a, x, t, tt, lane, st);
+  }
+}
+
+template <int NB, int THREADS>
+__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void attn_short_kernel(AttnArgs a, int n_seg, int item_rows) {
+  constexpr int D = 128, CH = 16, NW = THREADS / 64, LPB = kBKB * CH / THREADS, SLOT = kBKB * D;
+  __shared__ __attribute__((aligned(1024))) uint16_t kv[2 * NB * SLOT];
+  __shared__ __attribute__((aligned(16))) uint16_t stage[NW * 32 * 64];   // per wavefront 32 rows x 64 dims
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l32 = lane & 31, h = lane >> 5;
+  // this block's item: tile `tile` (item_rows queries) of the segments' tiles in order, and a head
+  int tile = blockIdx.x / a.H, seg = -1;
+  for (int s0 = 0; s0 < n_seg; s0 += 64) {
+    const int s = s0 + lane;
+    const int lq = s < n_seg ? a.cu_q[s + 1] - a.cu_q[s] : 0;
+    int incl = lq > 0 ? (lq + item_rows - 1) / item_rows : 0;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int y = __shfl_up(incl, o, 64);
+      if (lane >= o) incl += y;
+    }
+    const int total = __shfl(incl, 63, 64);
+    if (tile < total) {
+      const int before = __popcll(__ballot(incl <= tile));   // incl does not decrease: the lanes below
+      seg = s0 + before;
+      if (before > 0) tile -= __shfl(incl, before - 1, 64);
+      break;
+    }
+    tile -= total;
+  }
+  seg = __builtin_amdgcn_readfirstlane(seg);
+  tile = __builtin_amdgcn_readfirstlane(tile);
+  if (seg < 0) return;   // the grid covers the most tiles the call can have
+  ShortItem x;
+  x.head = blockIdx.x % a.H;
+  x.q0 = a.cu_q[seg] + tile * item_rows;
+  x.rows = min(item_rows, a.cu_q[seg + 1] - x.q0);
+  x.Lk = max(a.k_len ? a.k_len[seg] : a.cu_k[seg + 1] - a.cu_k[seg], 0);
+  const int k_beg = a.k_off ? a.k_off[seg] : a.cu_k[seg];
+  const int nb = (x.Lk + kBKB - 1) / kBKB;
+
+  // LDS read addresses and DMA lane offsets, as attn8_kernel's
+  const int krow = pi32(l32), ksw = swz4_k<CH>(krow);
+  const uint32_t kb = krow * D * 2 + (uint32_t)((h ^ (ksw & 1)) * 16 + 32 * (ksw >> 1));
+  const int r = lane & 15, g4 = lane >> 4;
+  const uint32_t vb = (16 * h + (r >> 2)) * D * 2 + (2 * (g4 & 1) + ((r >> 1) & 1)) * 16 + (r & 1) * 8 +
+                      64 * ((r >> 2) & 3);
+  const int64_t rs = a.ks;
+  uint32_t voffk[LPB], voffv[LPB];
+#pragma unroll
+  for (int n = 0; n < LPB; ++n) {
+    const int slot = n * THREADS + w * 64 + lane, row = slot / CH, phys = slot % CH;
+    voffk[n] = (uint32_t)(row * rs * 2 + (phys ^ swz4_k<CH>(row)) * 16);
+    voffv[n] = (uint32_t)(row * rs * 2 + (phys ^ swz4_v<CH>(row)) * 16);
+  }
+  const uint64_t kbase = (uint64_t)(a.k + (int64_t)k_beg * rs + x.head * D);
+  const uint64_t vbase = (uint64_t)(a.v + (int64_t)k_beg * rs + x.head * D);
+  const int32_t rb = (int32_t)rs * 2, bb = kBKB * rb, rem0 = x.Lk * rb - rb + D * 2;
+  const uint32_t m0w = lds_addr(kv) + (uint32_t)w * 64 * 16;
+  auto load_blocks = [&](int b0, int n) {   // key blocks b0 .. b0 + n - 1 into slots 0 .. n - 1 (rows past Lk: zeros)
+    for (int b = 0; b < n; ++b) {
+      const int blk = b0 + b;
+      const int32_t nrec = max(rem0 - blk * bb, 0);
+      dma_block<LPB>(kbase + (uint64_t)blk * (uint32_t)bb, nrec, voffk, m0w + b * SLOT * 2);
+      dma_block<LPB>(vbase + (uint64_t)blk * (uint32_t)bb, nrec, voffv, m0w + (NB + b) * SLOT * 2);
+    }
+  };
+  ShortLds ad;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    ad.k[k] = lds_addr(kv) + (kb ^ (32 * k));
+    asm volatile("" : "+v"(ad.k[k]));   // one register each: not re-derived from a base with larger offsets
+  }
+#pragma unroll
+  for (int db = 0; db < 4; ++db) {
+    ad.v[db] = lds_addr(kv) + NB * SLOT * 2 + (vb ^ (64 * db));
+    asm volatile("" : "+v"(ad.v[db]));
+  }
+  uint16_t* st = stage + w * 32 * 64;
+  load_blocks(0, min(nb, NB));
+  wait_loads_barrier<0>();
+  switch (nb <= NB ? nb : -1) {
+    case 1: short_tiles<1, NW>(a, x, ad, w, lane, st); return;
+    case 2: short_tiles<2, NW>(a, x, ad, w, lane, st); return;
+    case 3: short_tiles<3, NW>(a, x, ad, w, lane, st); return;
+    case 4: short_tiles<4, NW>(a, x, ad, w, lane, st); return;
+    default: break;
+  }
+  if constexpr (NB == 8) switch (nb <= NB ? nb : -1) {
+    case 5: short_tiles<5, NW>(a, x, ad, w, lane, st); return;
+    case 6: short_tiles<6, NW>(a, x, ad, w, lane, st); return;
+    case 7: short_tiles<7, NW>(a, x, ad, w, lane, st); return;
+    case 8: short_tiles<8, NW>(a, x, ad, w, lane, st); return;
+    default: break;
+  }
+  // no keys (O = 0, lse = -inf), or more of them than max_k said: block by block through slot 0
+  for (int t0 = 0; 32 * t0 < x.rows; t0 += NW) {
+    ShortTile t;
+    const uint16_t* qp = short_q(a, x, t0 + w, l32, h);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) t.q[k] = as_bf16x8(*(const u32x4*)(qp + 16 * k));
+    t.m = kMInit;
+    t.l = 0.0f;
+#pragma unroll
+    for (int db = 0; db < 4; ++db)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) t.acc[db][e] = 0.0f;
+    for (int b = 0; b < nb; ++b) {
+      __syncthreads();
+      load_blocks(b, 1);
+      wait_loads_barrier<0>();
+      short_chunk<1, false>(t, ad, 0, x.Lk - b * kBKB - 16 * h, a.c, nullptr);
+    }
+    short_store(a, x, t, t0 + w, lane, st);
+  }
+}
+
 typedef void (*AttnFn)(AttnArgs, int32_t*);
 
 // head_dim 128 runs the 64-query kernel (256-query items), head_dim 64 the 32-query kernel (128-query items)
@@ -1338,6 +1626,31 @@ int check_args(const or_varlen_args& x, const char* fn) {
   return 0;
 }
 
+// calls that attn_short_kernel runs: at most 256 keys per segment (K and V of a head in 128 KB of LDS), without the
+// options that only the ring kernels have (queries named by source row among them: a scene layer's calls, which give the
+// same bits with their values packed or read in place, stay on one kernel), and with few enough segments that finding one is cheap (256 segments of 10
+// queries x 24 heads: 172 -> 62 us; each further 64 cost every block another look at cu_q). Segments longer than max_k
+// says still come out right (streamed block by block for every tile).
+bool short_keys(const or_varlen_args& x) {
+  return x.D == 128 && x.max_k >= 1 && x.max_k <= kShortKeys && x.n_seg <= kShortSegs && !x.seg_q_src && !x.q_rope &&
+         !x.k_len_head && !x.v_tok && !x.k_tok;
+}
+
+int launch_short(const or_varlen_args& x, const AttnArgs& a, const DevInfo& di, hipStream_t st) {
+  const bool half = x.max_k <= kShortKeys / 2;
+  // queries per item: as many as leave four items per resident block, so that K / V are loaded for few items and the
+  // last round stays short (128 for every call made no difference at 211 200 queries, within 3%)
+  const int base = half ? 128 : 256;
+  const int64_t slots = (int64_t)di.cus * (half ? 2 : 1);
+  int rows = 8 * base;
+  while (rows > base && (int64_t)x.sum_q / rows * x.H < 4 * slots) rows /= 2;
+  const int64_t tiles = ((int64_t)x.sum_q + rows - 1) / rows + x.n_seg;
+  const dim3 grid((unsigned)(tiles * x.H));
+  if (half) hipLaunchKernelGGL((attn_short_kernel<4, 256>), grid, dim3(256), 0, st, a, x.n_seg, rows);
+  else hipLaunchKernelGGL((attn_short_kernel<8, 512>), grid, dim3(512), 0, st, a, x.n_seg, rows);
+  return check_hip(hipGetLastError(), "attn_short_kernel launch");
+}
+
 // planner + attention kernel (+ merge of key-split parts) on workspace `wsp`, laid out by ws_layout(..., cap)
 int launch_varlen(const or_varlen_args& x, void* wsp, int64_t cap, hipStream_t st) {
   if (x.sum_q == 0) return 0;
@@ -1378,6 +1691,7 @@ int launch_varlen(const or_varlen_args& x, void* wsp, int64_t cap, hipStream_t s
   a.H = x.H;
   a.scale = x.scale;
   a.c = x.scale * 1.4426950408889634f;
+  if (short_keys(x)) return launch_short(x, a, di, st);
   int32_t* ws = (int32_t*)wsp;
   const WsLayout wl = ws_layout(x.n_seg, x.sum_q, x.H, cap);
   a.v_tok = (const uint16_t*)x.v_tok;
