@@ -326,6 +326,10 @@ int or_frame_pool(const void* hs, int64_t n_rows, int32_t C, int64_t row_stride,
 int or_frame_select(const float* feats, int32_t n_frames, int32_t C, const int32_t* cand, int32_t n_cand, int32_t k,
                     int32_t iters, int32_t* reps, float* work, void* stream);
 
+/* or_frame_select with cand in host memory, each below min(n_frames, 65536): they travel with the launch. */
+int or_frame_select_host(const float* feats, int32_t n_frames, int32_t C, const int32_t* cand, int32_t n_cand,
+                         int32_t k, int32_t iters, int32_t* reps, float* work, void* stream);
+
 /* Bytes of device workspace or_memory_select needs: the normalised keys [H, B, D] fp32 and per-candidate arrays. */
 int64_t or_memory_select_workspace_size(int32_t B, int32_t H, int32_t D, int32_t M, int32_t iters);
 

@@ -82,6 +82,7 @@ SIGNATURES = {
     'or_rmsnorm_rope': (i32, [vp, vp, vp, vp, i64, i64, i64, i32, i32, ctypes.c_float, vp, vp, vp, i64, vp, vp, i64,
                               i64, vp]),
     'or_frame_pool': (i32, [vp, i64, i32, i64, i64, i32, i32, vp, vp, vp]),
+    'or_frame_select_host': (i32, [vp, i32, i32, vp, i32, i32, i32, vp, vp, vp]),
     'or_frame_select': (i32, [vp, i32, i32, vp, i32, i32, i32, vp, vp, vp]),
     'or_memory_select_workspace_size': (i64, [i32, i32, i32, i32, i32]),
     'or_memory_select': (i32, [vp, i32, vp, i64, i32, i32, i32, i32, vp, vp, i32, vp, vp, vp, i64, vp]),

@@ -7,8 +7,8 @@
 // centre (the first on ties). Here:
 //
 // - frame_pool_kernel: rows are frame-major (frame of row r = (row0 + r) / T, as the one-GPU processors build
-//   them), so a frame's rows are contiguous. One wavefront per (frame, 512-column block) adds them in row order:
-//   deterministic, unlike an atomic index_add_. Per lane, 8 consecutive columns in fp32.
+//   them), so a frame's rows are contiguous. One wavefront per (frame, 128 columns) adds them in row order:
+//   deterministic, unlike an atomic index_add_. Per lane, 2 consecutive columns in fp32.
 // - frame_select_kernel: the whole selection in one workgroup of 1024 threads, centres in LDS (k * C floats); no
 //   host round trip per iteration. Ties are broken towards the lower index, as torch.argmax does. A pass stops when
 //   the new centres equal the old ones exactly (torch.equal).
@@ -20,7 +20,7 @@ namespace onereel {
 
 namespace {
 
-constexpr int kPoolThreads = 256;
+constexpr int kPoolFly = 32;     // rows per batch of the pooling
 constexpr int kSelThreads = 1024;
 constexpr int kSelWaves = kSelThreads / 64;
 constexpr int kMaxCand = 1024;
@@ -35,53 +35,46 @@ struct PoolArgs {
   float* counts;     // [n_frames]
 };
 
-// grid: (groups of four 512-column blocks, frames); each wavefront covers 512 columns (64 lanes x 8) of one frame
-__global__ __launch_bounds__(kPoolThreads) void frame_pool_kernel(PoolArgs g) {
-  const int lane = threadIdx.x & 63;
-  const int cb = blockIdx.x * (kPoolThreads / 64) + (threadIdx.x >> 6);   // 512-column block
-  const int f = blockIdx.y;
-  const int col = cb * 512 + 8 * lane;
-  if (col >= g.C) return;
+// One wavefront per (frame, 128 columns): a lane owns two columns and adds the frame's rows in row order, so the sums
+// have the same bits whatever the launch. The chain of dependent additions is short (1590 rows: 3 us); what counts are
+// the bytes in flight, so a batch of kPoolFly rows is loaded while the batch before it is added.
+// HBM-bound: eight columns per lane with four rows in flight had 128 wavefronts on the chip and took 168 us for 32
+// frames x 1590 rows x 2048 columns (1.2 TB/s), now 65 us (3.2 TB/s; batches of 64: 69).
+__global__ __launch_bounds__(64) void frame_pool_kernel(PoolArgs g) {
+  const int f = blockIdx.y, col = blockIdx.x * 128 + 2 * threadIdx.x;
   int64_t r0 = (int64_t)f * g.T - g.row0, r1 = r0 + g.T;
   r0 = r0 < 0 ? 0 : r0;
   r1 = r1 > g.n_rows ? g.n_rows : r1;
-  float acc[8] = {};
-  int64_t r = r0;
-  // four rows in flight per lane, added in row order
-  for (; r + 4 <= r1; r += 4) {
-    u32x4 v[4];
+  if (r1 <= r0 || col >= g.C) return;
+  const uint16_t* p = g.hs + r0 * g.row_stride + col;
+  const int n = (int)(r1 - r0);
+  float a0 = 0.0f, a1 = 0.0f;
+  uint32_t v[2][kPoolFly];
+  auto load = [&](int b, uint32_t (&x)[kPoolFly]) {   // batch b, rows past the last repeat it
 #pragma unroll
-    for (int u = 0; u < 4; ++u) v[u] = *(const u32x4*)(g.hs + (r + u) * g.row_stride + col);
+    for (int u = 0; u < kPoolFly; ++u) x[u] = *(const uint32_t*)(p + (int64_t)min(b * kPoolFly + u, n - 1) * g.row_stride);
+  };
+  auto add = [&](int b, const uint32_t (&x)[kPoolFly]) {
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
-#pragma unroll
-      for (int p = 0; p < 4; ++p) {
-        acc[2 * p] += bf2f((uint16_t)(v[u][p] & 0xffffu));
-        acc[2 * p + 1] += bf2f((uint16_t)(v[u][p] >> 16));
+    for (int u = 0; u < kPoolFly; ++u)
+      if (b * kPoolFly + u < n) {
+        a0 += bf2f((uint16_t)(x[u] & 0xffffu));
+        a1 += bf2f((uint16_t)(x[u] >> 16));
       }
+  };
+  const int batches = (n + kPoolFly - 1) / kPoolFly;
+  load(0, v[0]);
+  for (int b = 0; b < batches; b += 2) {
+    load(min(b + 1, batches - 1), v[1]);
+    add(b, v[0]);
+    load(min(b + 2, batches - 1), v[0]);
+    add(b + 1, v[1]);
   }
-  for (; r < r1; ++r) {
-    const u32x4 v = *(const u32x4*)(g.hs + r * g.row_stride + col);
-#pragma unroll
-    for (int p = 0; p < 4; ++p) {
-      acc[2 * p] += bf2f((uint16_t)(v[p] & 0xffffu));
-      acc[2 * p + 1] += bf2f((uint16_t)(v[p] >> 16));
-    }
-  }
-  if (r1 <= r0) return;
   float* sp = g.sums + (int64_t)f * g.C + col;
-#pragma unroll
-  for (int e = 0; e < 8; ++e) sp[e] += acc[e];
-  if (cb == 0 && lane == 0) g.counts[f] += (float)(r1 - r0);
+  sp[0] += a0;
+  sp[1] += a1;
+  if (col == 0) g.counts[f] += (float)n;
 }
-
-struct SelectArgs {
-  const float* feats;      // [n_frames, C], rows L2-normalised
-  const int32_t* cand;     // [n_cand] candidate frames
-  int n_cand, C, k, iters;
-  int32_t* reps;           // [k] out: chosen frames ascending, -1 after them
-  float* work;             // [8, C] workspace
-};
 
 // butterfly sum over the 64 lanes by xor shuffles, the same in every lane
 __device__ __forceinline__ float wave_sum_xor(float v) {
@@ -90,104 +83,160 @@ __device__ __forceinline__ float wave_sum_xor(float v) {
   return v;
 }
 
-// first index of the maximum of v[0 .. n) (n <= kMaxCand); every thread of the block calls it
-__device__ int block_argmax(const float* v, int n, float* sv, int* si) {
-  const int tid = threadIdx.x;
+// the candidate frames of a selection, passed with the launch (no copy to the device ahead of it)
+struct CandTable {
+  uint16_t frame[kMaxCand];
+};
+
+struct SelectArgs {
+  const float* feats;      // [n_frames, C], rows L2-normalised
+  const int32_t* cand;     // [n_cand] candidate frames, or NULL: the table
+  int n_cand, C, k, iters;
+  int32_t* reps;           // [k] out: chosen frames ascending, -1 after them
+  float* work;             // [8, C] workspace
+};
+
+// two candidate rows against the first `live` (at most NQ) rows of `cv`, C floats apart: acc[i][q] is the lane's share of
+// row i . cv_q, over e = lane, lane + 64, ... in that order. Both rows' loads go out together, 16 steps at a time.
+template <int NQ>
+__device__ __forceinline__ void dots(const float* x0, const float* x1, const float* cv, int live, int C, int lane,
+                                     float (&acc)[2][NQ]) {
+  constexpr int FLY = 16;
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) acc[i][q] = 0.0f;
+  for (int e0 = lane; e0 < C; e0 += 64 * FLY) {
+    float a[FLY], b[FLY];
+#pragma unroll
+    for (int u = 0; u < FLY; ++u) {
+      const int e = min(e0 + 64 * u, C - 1);
+      a[u] = x0[e];
+      b[u] = x1[e];
+    }
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+      if (q >= live) break;
+#pragma unroll
+      for (int u = 0; u < FLY; ++u) {
+        const int e = e0 + 64 * u;
+        if (e < C) {
+          const float c = cv[q * C + e];
+          acc[0][q] += a[u] * c;
+          acc[1][q] += b[u] * c;
+        }
+      }
+    }
+  }
+}
+
+// first index of the maximum of v[0 .. n), over one wavefront (n >= 1; the same in every lane). NaN entries never win
+// over an earlier entry.
+__device__ __forceinline__ int wave_argmax(const float* v, int n, int lane) {
   float best = -INFINITY;
   int bi = 0x7fffffff;
-  for (int i = tid; i < n; i += kSelThreads)
-    if (bi == 0x7fffffff || v[i] > best) {   // ascending i per thread: its first maximum
+  for (int i = lane; i < n; i += 64)
+    if (bi == 0x7fffffff || v[i] > best) {   // ascending i per lane: its first maximum
       best = v[i];
       bi = i;
     }
-  sv[tid] = best;
-  si[tid] = bi;
-  __syncthreads();
-  for (int o = kSelThreads / 2; o > 0; o >>= 1) {
-    if (tid < o) {
-      const float b = sv[tid + o];
-      const int j = si[tid + o];
-      if (b > sv[tid] || (b == sv[tid] && j < si[tid])) {
-        sv[tid] = b;
-        si[tid] = j;
-      }
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) {
+    const float b = __shfl_xor(best, o, 64);
+    const int j = __shfl_xor(bi, o, 64);
+    if (b > best || (b == best && j < bi)) {
+      best = b;
+      bi = j;
     }
-    __syncthreads();
   }
-  const int r = si[0];
-  __syncthreads();
-  return r;
+  return bi < n ? bi : 0;
 }
 
-// dot product of candidate row n with a centre (LDS or global), reduced over the wavefront
-__device__ __forceinline__ float row_dot(const SelectArgs& g, int n, const float* cv, int lane) {
-  const float* x = g.feats + (int64_t)g.cand[n] * g.C;
-  float acc = 0.0f;
-  for (int e = lane; e < g.C; e += 64) acc += x[e] * cv[e];
-  return wave_sum_xor(acc);
-}
-
-__global__ __launch_bounds__(kSelThreads) void frame_select_kernel(SelectArgs g) {
-  extern __shared__ float smem[];
+// The whole choice in one workgroup: every pass is a few microseconds of dependent loads from the L2, so the passes are
+// few and each keeps many loads in flight: two candidate rows per wavefront and 16 steps of each at once, 16 rows of a
+// column at once in the member sums, and the similarities of the last assignment serve the medoids. Every sum keeps the
+// order of a plain loop over lanes and rows: in a cluster of two, both members are equally similar to their mean, so a
+// sum taken in another order would choose the other one.
+// 32 candidates x 2048 columns, 4 centres: 157 us (one 4-byte load at a time per thread, a pass over the candidates and
+// a block-wide argmax tree per medoid) -> 81 us.
+__global__ __launch_bounds__(kSelThreads) void frame_select_kernel(SelectArgs g, CandTable table) {
+  extern __shared__ __attribute__((aligned(16))) float smem[];
   float* c = smem;                  // [k, C] centres
   float* mrow = g.work;             // [8, C] means of the eight clusters being updated (global workspace)
   __shared__ float dv[kMaxCand];    // per-candidate scores
   __shared__ int z[kMaxCand];       // assignment
-  __shared__ float sv[kSelThreads];
-  __shared__ int si[kSelThreads];
+  __shared__ int cand[kMaxCand];
+  __shared__ float sv[8 * kSelWaves];
   __shared__ int centre[kMaxK];
   __shared__ int cnt[kMaxK];
   __shared__ int changed;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int nc = g.n_cand, C = g.C, k = g.k;
+  for (int n = tid; n < nc; n += kSelThreads) {
+    cand[n] = g.cand ? g.cand[n] : table.frame[n];
+    dv[n] = INFINITY;
+  }
+  if (tid == 0) centre[0] = 0;
+  __syncthreads();
+  auto row = [&](int n) { return g.feats + (int64_t)cand[min(n, nc - 1)] * C; };
 
   // farthest-point initialisation: centre 0 is candidate 0, then each time the candidate whose nearest chosen
   // centre is farthest (largest 1 - dot)
-  for (int n = tid; n < nc; n += kSelThreads) dv[n] = INFINITY;
-  if (tid == 0) centre[0] = 0;
-  __syncthreads();
   for (int m = 1; m < k; ++m) {
-    const float* xc = g.feats + (int64_t)g.cand[centre[m - 1]] * C;
-    for (int n = w; n < nc; n += kSelWaves) {
-      const float d = 1.0f - row_dot(g, n, xc, lane);
-      if (lane == 0) dv[n] = fminf(dv[n], d);
+    const float* xc = row(centre[m - 1]);
+    for (int n = 2 * w; n < nc; n += 2 * kSelWaves) {
+      float acc[2][1];
+      dots<1>(row(n), row(n + 1), xc, 1, C, lane, acc);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const float d = 1.0f - wave_sum_xor(acc[i][0]);
+        if (lane == 0 && n + i < nc) dv[n + i] = fminf(dv[n + i], d);
+      }
     }
     __syncthreads();
-    const int a = block_argmax(dv, nc, sv, si);
-    if (tid == 0) centre[m] = a;
+    if (w == 0) {
+      const int a = wave_argmax(dv, nc, lane);
+      if (lane == 0) centre[m] = a;
+    }
     __syncthreads();
   }
-  for (int e = tid; e < k * C; e += kSelThreads) c[e] = g.feats[(int64_t)g.cand[centre[e / C]] * C + e % C];
+  for (int i = 0; i < k; ++i) {
+    const float* x = row(centre[i]);
+    for (int e = tid; e < C; e += kSelThreads) c[i * C + e] = x[e];
+  }
   __syncthreads();
 
   // k-means: z = the most similar centre (first on ties); centre i = normalize(mean of its members), unchanged when
   // it has none; stop when no centre changed. After the loop z belongs to the final centres. Centres are taken eight
   // at a time, so that a candidate row is read once per eight dot products and the member sums of eight clusters
-  // accumulate in one pass over the rows (in row order).
+  // accumulate in one pass over the rows (in row order). dv: each candidate's similarity to its centre.
   for (int it = 0;; ++it) {
-    for (int n = w; n < nc; n += kSelWaves) {
-      const float* x = g.feats + (int64_t)g.cand[n] * C;
-      float best = 0.0f;
-      int bi = 0;
+    for (int n = 2 * w; n < nc; n += 2 * kSelWaves) {
+      float best[2] = {0.0f, 0.0f};
+      int bi[2] = {0, 0};
       for (int i0 = 0; i0 < k; i0 += 8) {
-        float acc[8] = {};
-        for (int e = lane; e < C; e += 64) {
-          const float xv = x[e];
-#pragma unroll
-          for (int q = 0; q < 8; ++q)
-            if (i0 + q < k) acc[q] += xv * c[(i0 + q) * C + e];
-        }
+        float acc[2][8];
+        dots<8>(row(n), row(n + 1), c + i0 * C, k - i0, C, lane, acc);
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
           if (i0 + q >= k) break;
-          const float d = wave_sum_xor(acc[q]);
-          if (i0 + q == 0 || d > best) {
-            best = d;
-            bi = i0 + q;
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            const float d = wave_sum_xor(acc[i][q]);
+            if (i0 + q == 0 || d > best[i]) {
+              best[i] = d;
+              bi[i] = i0 + q;
+            }
           }
         }
       }
-      if (lane == 0) z[n] = bi;
+      if (lane == 0)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+          if (n + i < nc) {
+            z[n + i] = bi[i];
+            dv[n + i] = best[i];
+          }
     }
     if (tid < k) cnt[tid] = 0;
     if (tid == 0) changed = 0;
@@ -199,13 +248,16 @@ __global__ __launch_bounds__(kSelThreads) void frame_select_kernel(SelectArgs g)
       float part[8] = {};
       for (int e = tid; e < C; e += kSelThreads) {
         float sum[8] = {};
-        for (int n = 0; n < nc; ++n) {
-          const int zi = z[n] - i0;     // the same for every thread: a uniform branch
-          if (zi < 0 || zi >= 8) continue;
-          const float v = g.feats[(int64_t)g.cand[n] * C + e];
+        for (int n0 = 0; n0 < nc; n0 += 16) {
+          float v[16];
 #pragma unroll
-          for (int q = 0; q < 8; ++q)
-            if (zi == q) sum[q] += v;
+          for (int u = 0; u < 16; ++u) v[u] = row(n0 + u)[e];
+#pragma unroll
+          for (int u = 0; u < 16; ++u) {
+            const int zi = n0 + u < nc ? z[n0 + u] - i0 : -1;   // the same for every thread
+#pragma unroll
+            for (int q = 0; q < 8; ++q) sum[q] += zi == q ? v[u] : 0.0f;
+          }
         }
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
@@ -217,6 +269,7 @@ __global__ __launch_bounds__(kSelThreads) void frame_select_kernel(SelectArgs g)
       }
 #pragma unroll
       for (int q = 0; q < 8; ++q) {
+        if (i0 + q >= k) break;
         const float p = wave_sum_xor(part[q]);
         if (lane == 0) sv[q * kSelWaves + w] = p;
       }
@@ -224,6 +277,7 @@ __global__ __launch_bounds__(kSelThreads) void frame_select_kernel(SelectArgs g)
       for (int q = 0; q < 8 && i0 + q < k; ++q) {
         if (cnt[i0 + q] == 0) continue;   // no members: the centre stays
         float t = 0.0f;
+#pragma unroll
         for (int u = 0; u < kSelWaves; ++u) t += sv[q * kSelWaves + u];
         const float nrm = fmaxf(sqrtf(t), 1e-12f);
         float* ci = c + (i0 + q) * C;
@@ -235,39 +289,41 @@ __global__ __launch_bounds__(kSelThreads) void frame_select_kernel(SelectArgs g)
       }
       __syncthreads();
     }
-    if (!changed) break;   // z was computed from these (unchanged) centres
+    if (!changed) break;   // z and dv were computed from these (unchanged) centres
     __syncthreads();
   }
 
-  // medoid of each non-empty cluster: the member most similar to its centre, the first on ties
-  for (int i = 0; i < k; ++i) {
-    for (int n = w; n < nc; n += kSelWaves) {
-      float d = -INFINITY;
-      if (z[n] == i) d = row_dot(g, n, c + i * C, lane);
-      if (lane == 0) dv[n] = d;
-    }
-    if (tid == 0) changed = 0;
-    __syncthreads();
-    for (int n = tid; n < nc; n += kSelThreads)
-      if (z[n] == i) changed = 1;
-    __syncthreads();
-    const int any = changed;
-    const int a = block_argmax(dv, nc, sv, si);
-    if (tid == 0) centre[i] = any ? g.cand[a] : -1;
-    __syncthreads();
-  }
-  if (tid == 0) {
-    int out[kMaxK];
-    int n = 0;
-    for (int i = 0; i < k; ++i)
-      if (centre[i] >= 0) out[n++] = centre[i];
-    for (int a = 1; a < n; ++a)
-      for (int b = a; b > 0 && out[b - 1] > out[b]; --b) {
-        const int t = out[b];
-        out[b] = out[b - 1];
-        out[b - 1] = t;
+  // medoid of each non-empty cluster: the member most similar to its centre, the first on ties (a wavefront per cluster)
+  for (int i = w; i < k; i += kSelWaves) {
+    float best = -INFINITY;
+    int bi = 0x7fffffff;
+    for (int n = lane; n < nc; n += 64)
+      if (z[n] == i && (bi == 0x7fffffff || dv[n] > best)) {
+        best = dv[n];
+        bi = n;
       }
-    for (int i = 0; i < k; ++i) g.reps[i] = i < n ? out[i] : -1;
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) {
+      const float b = __shfl_xor(best, o, 64);
+      const int j = __shfl_xor(bi, o, 64);
+      if (j != 0x7fffffff && (bi == 0x7fffffff || b > best || (b == best && j < bi))) {
+        best = b;
+        bi = j;
+      }
+    }
+    if (lane == 0) centre[i] = bi < nc ? cand[bi] : -1;
+  }
+  __syncthreads();
+  // ascending, -1 after the last: a frame's place is the number of smaller ones
+  if (tid < k) {
+    const int f = centre[tid];
+    int place = 0, found = 0;
+    for (int i = 0; i < k; ++i) {
+      place += centre[i] >= 0 && (centre[i] < f || (centre[i] == f && i < tid));
+      found += centre[i] >= 0;
+    }
+    if (f >= 0) g.reps[place] = f;
+    if (tid >= found) g.reps[tid] = -1;
   }
 }
 
@@ -288,21 +344,20 @@ extern "C" int or_frame_pool(const void* hs, int64_t n_rows, int32_t C, int64_t 
                     n_frames);
   if (((uintptr_t)hs & 15u) || row_stride % 8) return fail_arg("or_frame_pool: hs must be 16-byte aligned rows");
   PoolArgs g{(const uint16_t*)hs, n_rows, row_stride, row0, C, T, n_frames, sums, counts};
-  const int col_blocks = (C + 512 - 1) / 512;
-  const dim3 grid((unsigned)((col_blocks + 3) / 4), (unsigned)n_frames);
-  hipLaunchKernelGGL(frame_pool_kernel, grid, dim3(kPoolThreads), 0, (hipStream_t)stream, g);
+  hipLaunchKernelGGL(frame_pool_kernel, dim3((unsigned)((C + 127) / 128), (unsigned)n_frames), dim3(64), 0,
+                     (hipStream_t)stream, g);
   return check_hip(hipGetLastError(), "frame_pool_kernel launch");
 }
 
-extern "C" int or_frame_select(const float* feats, int32_t n_frames, int32_t C, const int32_t* cand, int32_t n_cand,
-                               int32_t k, int32_t iters, int32_t* reps, float* work, void* stream) {
+// the candidates from the device (cand) or from the host (table; cand NULL)
+static int launch_select(const float* feats, int n_frames, int C, const int32_t* cand, const CandTable& table, int n_cand,
+                         int k, int iters, int32_t* reps, float* work, void* stream) {
   if (C < 1 || n_frames < 1 || n_cand < 1 || n_cand > kMaxCand || k < 1 || k > kMaxK || k > n_cand || iters < 0)
     return fail_arg("or_frame_select: need C >= 1, 1 <= n_cand <= %d and 1 <= k <= min(n_cand, %d) (n_cand=%d k=%d)",
                     kMaxCand, kMaxK, n_cand, k);
   if ((int64_t)k * C > kMaxCentreFloats)
     return fail_arg("or_frame_select: k * C = %lld floats of centres exceed %d of LDS", (long long)k * C,
                     kMaxCentreFloats);
-  if (!feats || !cand || !reps || !work) return fail_arg("or_frame_select: feats, cand, reps and work are required");
   SelectArgs g{feats, cand, n_cand, C, k, iters, reps, work};
   const size_t lds = (size_t)k * C * sizeof(float);
   static thread_local bool attr = false;
@@ -313,6 +368,25 @@ extern "C" int or_frame_select(const float* feats, int32_t n_frames, int32_t C, 
       return rc;
     attr = true;
   }
-  hipLaunchKernelGGL(frame_select_kernel, dim3(1), dim3(kSelThreads), lds, (hipStream_t)stream, g);
+  hipLaunchKernelGGL(frame_select_kernel, dim3(1), dim3(kSelThreads), lds, (hipStream_t)stream, g, table);
   return check_hip(hipGetLastError(), "frame_select_kernel launch");
+}
+
+extern "C" int or_frame_select(const float* feats, int32_t n_frames, int32_t C, const int32_t* cand, int32_t n_cand,
+                               int32_t k, int32_t iters, int32_t* reps, float* work, void* stream) {
+  if (!feats || !cand || !reps || !work) return fail_arg("or_frame_select: feats, cand, reps and work are required");
+  return launch_select(feats, n_frames, C, cand, CandTable{}, n_cand, k, iters, reps, work, stream);
+}
+
+extern "C" int or_frame_select_host(const float* feats, int32_t n_frames, int32_t C, const int32_t* cand,
+                                    int32_t n_cand, int32_t k, int32_t iters, int32_t* reps, float* work,
+                                    void* stream) {
+  if (!feats || !cand || !reps || !work) return fail_arg("or_frame_select_host: feats, cand, reps and work are required");
+  CandTable table{};
+  for (int i = 0; i < n_cand && i < kMaxCand; ++i) {
+    if (cand[i] < 0 || cand[i] >= n_frames || cand[i] > 0xffff)
+      return fail_arg("or_frame_select_host: candidate frame %d outside [0, min(%d, 65536))", cand[i], n_frames);
+    table.frame[i] = (uint16_t)cand[i];
+  }
+  return launch_select(feats, n_frames, C, nullptr, table, n_cand, k, iters, reps, work, stream);
 }

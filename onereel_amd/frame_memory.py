@@ -159,9 +159,11 @@ class FrameMemory:
         if not self.sums:
             return
         layers = sorted(self.sums)
-        sums = torch.stack([self.sums[layer] for layer in layers])
-        counts = torch.stack([self.counts[layer] for layer in layers])
+        sums = [self.sums[layer] for layer in layers]
+        counts = [self.counts[layer] for layer in layers]
         self.sums, self.counts = {}, {}
+        # one layer's sums as they are, several stacked
+        sums, counts = (x[0][None] if len(x) == 1 else torch.stack(x) for x in (sums, counts))
         feats = F.normalize(sums / counts.clamp_min(1)[..., None], dim=-1)
         if self.per_layer:
             self.pending = {layer: self.select(f) for layer, f in zip(layers, feats)}
@@ -182,9 +184,13 @@ class FrameMemory:
             raise L.HipValueError(f'candidate frames outside [0, {n_frames})')
         x = feats.to(torch.float32).contiguous()
         dev = x.device
-        ct = torch.tensor(cand, dtype=torch.int32, device=dev)
         reps = torch.empty(k, dtype=torch.int32, device=dev)
         work = torch.empty(8, C, dtype=torch.float32, device=dev)
-        L.check(L.lib().or_frame_select(x.data_ptr(), n_frames, C, ct.data_ptr(), len(cand), k, self.iters,
-                                        reps.data_ptr(), work.data_ptr(), L.stream_handle(dev)), 'or_frame_select')
+        if n_frames <= 65536:
+            # the candidates travel with the launch
+            fn, ct = L.lib().or_frame_select_host, torch.tensor(cand, dtype=torch.int32)
+        else:
+            fn, ct = L.lib().or_frame_select, torch.tensor(cand, dtype=torch.int32, device=dev)
+        L.check(fn(x.data_ptr(), n_frames, C, ct.data_ptr(), len(cand), k, self.iters, reps.data_ptr(),
+                   work.data_ptr(), L.stream_handle(dev)), 'or_frame_select')
         return [int(r) for r in reps.cpu().tolist() if r >= 0]
