@@ -210,5 +210,4 @@ class Processor:
             pieces = [(j, lo * T, hi * T) for j, (lo, hi) in enumerate(lay.ranges)]
             mem.plans[pk] = frame_plan(lay, T, torch.arange(Sq), k.shape[0], pieces, ctx.text_ranges(),
                                        set(range(lay.n_scenes)), Sq, q.device)
-        out = mem((self.layer, ctx.cond()), torch.cat([q, eq]), torch.cat([k, ek]), torch.cat([v, ev]), mem.plans[pk])
-        return out[:Sq], out[Sq:]
+        return mem.with_text((self.layer, ctx.cond()), q, k, v, eq, ek, ev, mem.plans[pk])

@@ -214,6 +214,7 @@ class _Static:
         self.in_place = (all(f is not None for f in first) and spans[0][0] >= 0 and spans[-1][1] <= Sq and
                          all(a[1] <= b[0] for a, b in zip(spans, spans[1:])))
         self.covers_all = self.in_place and sum(qlen) == Sq
+        self.spans = spans if self.in_place else None      # the pieces' query rows, ascending
         t32 = lambda x: torch.tensor(x, dtype=torch.int32, device=device)
         cu = [0]
         for _ in range(H):
@@ -237,6 +238,7 @@ class _Static:
         if lo < 0:
             raise L.HipValueError(f'plan key rows include {lo}: rows must be >= 0')
         self.max_key_row = max(int(local.max()) if local.numel() else -1, int(p.cand.max()))
+        self.max_cand = int(p.cand.max()) if p.cand.numel() else -1
         self.local = local.to(torch.int64)
         # a piece that does not read the memory and has the same local rows as another piece (a scene's sentence
         # queries beside its video queries) reads that piece's local rows in place: its keys are their slot's first
@@ -267,12 +269,20 @@ class _Static:
         self._slots = {}
         self.device = device
 
-    def multi_head(self, M: int):
+    def covers(self, lo: int, hi: int) -> bool:
+        """whether the pieces' query rows cover [lo, hi) (in_place plans)"""
+        at = lo
+        for a, b in self.spans:
+            if a <= at < b:
+                at = b
+        return at >= hi
+
+    def multi_head(self, M: int, end: int):
         """the multi-head form's per-M tables: per piece its packed row offset (k_off), largest key count (k_len),
-        in-place run (lead: whole 32-key blocks of keys and values from token row v_row); the pack job of the local
-        rows past the run (src, dst), and the packed row count. A piece that shares another's local rows gets that
-        piece's offset and run."""
-        key = ('mh', M)
+        in-place run (lead: whole 32-key blocks of keys and values from token row v_row, all of them below row `end`,
+        the first buffer's rows); the pack job of the local rows past the run (src, dst), and the packed row count. A
+        piece that shares another's local rows gets that piece's offset and run."""
+        key = ('mh', M, end)
         if key not in self._slots:
             n, lens = self.n, self.lens
             starts = [0]
@@ -293,9 +303,9 @@ class _Static:
                 rows = local[starts[i]:starts[i + 1]]
                 run = 0
                 if len(rows):
-                    step = (rows - rows[0]) == torch.arange(len(rows))
+                    step = ((rows - rows[0]) == torch.arange(len(rows))) & (rows < end)
                     run = len(rows) if bool(step.all()) else int((~step).nonzero()[0])
-                    v_row[i] = int(rows[0])
+                    v_row[i] = int(rows[0]) if run else 0
                 v_lead[i] = run // L.KEY_BLOCK * L.KEY_BLOCK
                 if self.share[i] is None:
                     src += rows[v_lead[i]:].tolist()
@@ -369,7 +379,7 @@ class MemoryAttention:
         rep, valid = self.memory._select(key, k, st.cand32, st.B, H, D)
         M = rep.shape[1]
         if st.in_place and not self.head_major:
-            return self._multi_head(st, q, k, v, rep, valid, M)
+            return self._multi_head(st, q, k, v, rep, valid, M)[0]
         k_off, kidx = st.slots(M)
         k_len = torch.empty(st.n * H, dtype=torch.int32, device=dev)
         L.check(L.lib().or_memory_index(rep.data_ptr(), valid.data_ptr(), st.cand64.data_ptr(), st.owner64.data_ptr(),
@@ -391,14 +401,35 @@ class MemoryAttention:
         scatter_rows(o, st.qidx, out.view(Sq * H, 1, D), check=False)
         return out
 
-    def _multi_head(self, st: _Static, q, k, v, rep, valid, M: int) -> torch.Tensor:
+    def with_text(self, key, q, k, v, eq, ek, ev, p: Plan):
+        """the call on q, k, v [N, H, D] (video rows) and eq, ek, ev [Le, H, D] (text rows) for a plan whose buffers are
+        the video rows followed by the text rows -> (video out, text out). Both parts are read where they are when the
+        multi-head form runs and they can be (copying q, k and v of 50 880 rows x 16 heads x 128 end to end took 455 of
+        the 480p call's 5218 us, now 4754); anything else is copied end to end first."""
+        N, Le = q.shape[0], eq.shape[0]
+        parts = (q, k, v, eq, ek, ev)
+        H, D = q.shape[-2:]
+        if (not self.head_major and N > 0 and Le > 0 and q.dim() == 3 and k.shape == q.shape and v.shape == q.shape and
+                eq.shape == ek.shape == ev.shape == (Le, H, D) and
+                all(x.is_cuda and x.device == q.device and x.dtype == torch.bfloat16 and x.stride() == (H * D, D, 1) and
+                    x.data_ptr() % 16 == 0 for x in parts)):
+            st = self._tables(p, H, N + Le, q.device)
+            if st.in_place and st.n * H <= 4096 and st.max_key_row < N + Le and st.max_cand < N:
+                rep, valid = self.memory._select(key, k, st.cand32, st.B, H, D)
+                return self._multi_head(st, q, k, v, rep, valid, rep.shape[1], (eq, ek, ev))
+        out = self(key, torch.cat([q, eq]), torch.cat([k, ek]), torch.cat([v, ev]), p)
+        return out[:N], out[N:]
+
+    def _multi_head(self, st: _Static, q, k, v, rep, valid, M: int, text=None):
         """every piece one multi-head segment: its local keys (the leading run of token rows, whole key blocks of it,
         read in place from k / v, the rest packed as whole rows) then, per head, that head's representatives of the
-        other scenes in its own head slot"""
+        other scenes in its own head slot. text: (eq, ek, ev), the rows after those of q, k and v. Returns the outputs
+        of q's rows and of the text's (None without)."""
         Sq, H, D = q.shape
         Lk = k.shape[0]
         dev = q.device
-        n, mh = st.n, st.multi_head(M)
+        n, mh = st.n, st.multi_head(M, Lk)
+        eq, ek, ev = text or (None, None, None)
         fsrc = torch.empty(n * H * M, dtype=torch.int32, device=dev)
         fdst = torch.empty_like(fsrc)
         k_len_head = torch.empty(n * H, dtype=torch.int32, device=dev)
@@ -413,10 +444,14 @@ class MemoryAttention:
         # local rows past the in-place run (checked once per plan), then the representatives (rows of the checked
         # candidates), one head each
         if mh['src'].numel():
-            pack_job(k, v, mh['src'], mh['dst'], kp, vp)
+            pack_job(k, v, mh['src'], mh['dst'], kp, vp, text=text and (ek, ev))
         pack_job(k.view(Lk * H, 1, D), v.view(Lk * H, 1, D), fsrc, fdst, kp.view(R * H, 1, D), vp.view(R * H, 1, D))
-        out = torch.empty_like(q) if st.covers_all else torch.zeros_like(q)
+        # rows outside the plan's queries are zero
+        out = torch.empty_like(q) if st.covers_all or st.covers(0, Sq) else torch.zeros_like(q)
+        out_text = None
+        if text:
+            out_text = torch.empty_like(eq) if st.covers_all else torch.zeros_like(eq)
         varlen(q, kp, vp, st.cu_piece, None, st.max_q, mh['max_k'], k_off=mh['k_off'], k_len=mh['k_len'], out=out,
                seg_q_src=st.first_q, n_q_video=Sq, sum_q=sum(st.qlen), v_tok=v, v_lead=mh['lead'],
-               v_row=mh['v_row'], k_tok=k, k_lead=mh['lead'], k_len_head=k_len_head)
-        return out
+               v_row=mh['v_row'], k_tok=k, k_lead=mh['lead'], k_len_head=k_len_head, q_text=eq, o_text=out_text)
+        return out, out_text

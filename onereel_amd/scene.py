@@ -222,13 +222,14 @@ def n_seg_of(cu_q: torch.Tensor) -> int:
     return cu_q.numel() - 1
 
 
-def pack_job(k, v, src, dst, k_out, v_out, v_src=None):
+def pack_job(k, v, src, dst, k_out, v_out, v_src=None, text=None):
     """one or_pack_layer launch without RoPE: packed row dst[r] of k_out / v_out = row src[r] of k / v (nothing for
     src[r] < 0; values from row v_src[r] when given, none where it is < 0). k, v, k_out, v_out: [rows, H, D] bf16 with
-    contiguous rows; the index arrays are int32 GPU tensors whose rows the caller has checked."""
+    contiguous rows; text: (k, v) rows alike that follow those of k and v; the index arrays are int32 GPU tensors whose
+    rows the caller has checked."""
     H, D = k.shape[1], k.shape[2]
-    _check_bf16(k, v, k_out, v_out)
-    for t in (k, v, k_out, v_out):
+    _check_bf16(k, v, k_out, v_out, *(text or ()))
+    for t in (k, v, k_out, v_out, *(text or ())):
         if not t.is_contiguous():
             raise L.HipValueError('pack_job takes contiguous [rows, H, D] tensors')
     for t in (src, dst, v_src):
@@ -240,6 +241,8 @@ def pack_job(k, v, src, dst, k_out, v_out, v_src=None):
         H * D, k.shape[0]
     a.k_src, a.v_src, a.k_dst, a.n_keys = src.data_ptr(), L.ptr(v_src), dst.data_ptr(), src.numel()
     a.k_out, a.v_out, a.H, a.D = k_out.data_ptr(), v_out.data_ptr(), H, D
+    if text:
+        a.k_text, a.v_text = text[0].data_ptr(), text[1].data_ptr()
     L.check(L.lib().or_pack_layer(ctypes.byref(a), L.stream_handle(k.device)), 'or_pack_layer')
 
 
