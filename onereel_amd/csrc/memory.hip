@@ -7,20 +7,26 @@
 // cluster sums, a host read per iteration for the convergence test, stable sorts for the tie-break.
 //
 // Here, per call:
-//   prep     one wavefront per (candidate, head): the key row (bf16 or fp32) in fp32, x = row / max(|row|, 1e-12),
-//            |x|^2; x stored [H, B, D] fp32. A cold start copies the evenly spaced candidates into the centroids.
-//   assign   per (64-candidate tile, head): dot products x . c by fp32 MFMA (v_mfma_f32_16x16x4_f32, the centroids
-//            in LDS), d = |x|^2 - 2 x . c + |c|^2, the nearest centroid (the lowest index on equal distances).
-//   group    one workgroup per head: a stable counting sort of the candidates by cluster (ascending candidate
-//            within a cluster), so that every later sum has a fixed order.
-//   update   per (cluster, head): the mean of the members in that order (fp32), or the old centroid when the
-//            cluster is empty; a flag records whether any centroid moved.
+//   prep     one wavefront per (candidate, 16 heads): inv = 1 / max(|row|, 1e-12) and |x|^2 of x = row * inv in fp32. bf16
+//            keys are left where they are and x is formed again from row and inv wherever it is used (the same fp32
+//            product; half the bytes of a stored x); fp32 keys are stored as x [H, B, D].
+//   start    |c|^2 of the centroids; a cold start first copies the evenly spaced candidates into them.
+//   assign   dot products x . c by fp32 MFMA (v_mfma_f32_16x16x4_f32), d = |x|^2 - 2 x . c + |c|^2, the nearest centroid
+//            (the lowest index on equal distances).
+//   update   per cluster: the mean of its members in ascending order (fp32, four partial sums), or the old centroid when
+//            the cluster is empty; a flag per head records whether any of its centroids moved.
 //   medoid   one workgroup per head: per non-empty cluster, in cluster order, the member nearest its centroid (the
 //            lowest candidate on equal distances) -> rep[h, r] (int64) and valid[h, r] = 1, then zeros.
-// assign / group / update of iteration it > 0 return at once when iteration it - 1 moved no centroid (a fixed point:
-// every later iteration would give the same assignment), so the host launches all passes without reading anything
-// back, and the result equals a loop that stops at convergence.
+// assign / update of iteration it > 0 return at once for the heads whose centroids iteration it - 1 did not move (a
+// fixed point: every later iteration would give the same assignment), so the host launches all passes without reading
+// anything back, and the result equals a loop that stops at convergence. A pass that finds nothing to do costs its
+// launch, so the grids are about two blocks per CU whatever the sizes.
+// Measured, 12 720 candidates x 16 heads x 128, M = 128: prep 49 -> 12.5 us, an assign 97 -> 79, an update 37 -> 25 (and a
+// counting sort of the candidates ahead of it 25 -> 0: every update block finds its clusters' members itself), medoids
+// 22 -> 12. 2340 candidates, first pass of a request: assign 23.5 -> 18, sort and update 17 to 35 -> 9 to 13.
 #include <math.h>
+
+#include <algorithm>
 
 #include "common.h"
 
@@ -28,11 +34,15 @@ namespace onereel {
 
 namespace {
 
-constexpr int kMaxClusters = 1024;  // M of one call (counting-sort table in LDS)
+constexpr int kMaxClusters = 1024;  // M of one call (one thread of the medoid kernel each)
 constexpr int kAssignThreads = 256;  // 4 wavefronts
-constexpr int kAssignRows = 64;      // candidates per assign block: 4 wavefronts x 16
-constexpr int kCChunk = 128;        // centroids per LDS chunk in assign
-constexpr int kCPitch = 132;        // floats per centroid row in LDS (padding spreads 16 rows over the banks)
+constexpr int kAssignTiles = 32;     // 16-candidate tiles per assign block at most (their results wait in LDS)
+constexpr int kPassBlocks = 512;     // blocks of an assign pass: two per CU
+constexpr int kUpdThreads = 512;
+constexpr int kUpdClusters = kUpdThreads / 128;   // clusters per update block
+constexpr int kUpdPer = 8;           // assignments per thread and chunk of an update block
+constexpr int kUpdChunk = kUpdThreads * kUpdPer;  // candidates looked at at once
+constexpr int kUpdFly = 16;          // member rows in flight per thread
 
 typedef float f32x4v __attribute__((ext_vector_type(4)));
 
@@ -41,24 +51,17 @@ struct SelArgs {
   const int32_t* rows;      // [B] row of each candidate in keys (NULL: candidate b is row b)
   int64_t stride;           // elements between consecutive rows of keys
   int B, H, D, M, fp32_in, iters;
-  float* X;                 // [H, B, D] normalised keys
+  float* X;                 // [H, B, D] normalised keys (fp32 keys only)
+  float* inv;               // [H, B] 1 / max(|key|, 1e-12)
   float* xx;                // [H, B] |x|^2
   float* C;                 // [H, M, D] centroids (in / out)
   float* cc;                // [H, M] |c|^2 of the current centroids
   int32_t* z;               // [H, B] cluster of each candidate
   float* dist;              // [H, B] its squared distance to that centroid
-  int32_t* order;           // [H, B] candidates grouped by cluster, ascending within a cluster
-  int32_t* start;           // [H, M + 1] group offsets into order
-  int32_t* moved;           // [iters + 1] moved[it] != 0: iteration it changed a centroid
+  int32_t* moved;           // [iters + 1, H] moved[it, h] != 0: iteration it changed a centroid of head h
   int64_t* rep;             // [H, M]
   uint8_t* valid;           // [H, M]
 };
-
-__device__ __forceinline__ float wave_sum64(float v) {
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
-}
 
 // ------------------------------------------------------------------------------------------------------------------
 // prep: one wavefront per (candidate b, group of 64 / LPH heads); LPH = D / 32 lanes per head, 32 consecutive elements
@@ -70,7 +73,7 @@ __global__ __launch_bounds__(256) void mem_prep_kernel(SelArgs g, int n_moved) {
   const int b = blockIdx.x * 4 + (threadIdx.x >> 6);
   const int h = blockIdx.y * HPW + lane / LPH, part = lane % LPH;
   if (blockIdx.x == 0 && blockIdx.y == 0)
-    for (int i = threadIdx.x; i < n_moved; i += 256) g.moved[i] = 1;   // until an update says otherwise
+    for (int i = threadIdx.x; i < n_moved; i += 256) g.moved[i] = 0;   // until an update says otherwise
   if (b >= g.B) return;
   const bool live = h < g.H;
   const int64_t row = g.rows ? g.rows[b] : b;
@@ -111,10 +114,15 @@ __global__ __launch_bounds__(256) void mem_prep_kernel(SelArgs g, int n_moved) {
 #pragma unroll
   for (int o = 1; o < LPH; o <<= 1) q += __shfl_xor(q, o, 64);
   if (!live) return;
-  f32x4v* x = (f32x4v*)(g.X + ((int64_t)h * g.B + b) * D + 32 * part);
+  if (g.fp32_in) {
+    f32x4v* x = (f32x4v*)(g.X + ((int64_t)h * g.B + b) * D + 32 * part);
 #pragma unroll
-  for (int k = 0; k < 8; ++k) x[k] = f32x4v{v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]};
-  if (part == 0) g.xx[(int64_t)h * g.B + b] = q;
+    for (int k = 0; k < 8; ++k) x[k] = f32x4v{v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]};
+  }
+  if (part == 0) {
+    g.inv[(int64_t)h * g.B + b] = inv;
+    g.xx[(int64_t)h * g.B + b] = q;
+  }
 }
 
 // |c|^2 of a centroid held one element per thread (threads 0..D-1 of a 128-thread group), summed by a fixed tree in
@@ -138,7 +146,14 @@ __global__ __launch_bounds__(128) void mem_start_kernel(SelArgs g, const int32_t
   float* dst = g.C + ((int64_t)h * g.M + i) * g.D;
   float c = 0.0f;
   if (d < g.D) {
-    c = init ? g.X[((int64_t)h * g.B + init[i]) * g.D + d] : dst[d];
+    if (!init) {
+      c = dst[d];
+    } else if (g.fp32_in) {
+      c = g.X[((int64_t)h * g.B + init[i]) * g.D + d];
+    } else {
+      const int64_t row = g.rows ? g.rows[init[i]] : init[i];
+      c = bf2f(((const uint16_t*)g.keys)[row * g.stride + (int64_t)h * g.D + d]) * g.inv[(int64_t)h * g.B + init[i]];
+    }
     if (init) dst[d] = c;
   }
   const float n2 = centroid_norm2(c, d, g.D, red);
@@ -146,296 +161,380 @@ __global__ __launch_bounds__(128) void mem_start_kernel(SelArgs g, const int32_t
 }
 
 // ------------------------------------------------------------------------------------------------------------------
-// assign: block (tile, h) takes candidates [64 tile, 64 tile + 64); wavefront w the 16 from 64 tile + 16 w. Two
-// blocks per CU (68 KB of LDS each), two wavefronts per SIMD.
-// MFMA 16x16x4 f32: lane l supplies A[l % 16][l / 16] and B[l / 16][l % 16] and holds D[4 (l / 16) + r][l % 16].
-// The reduction dimension is visited in the order d = (l / 16) * (D / 4) + s at step s (any order of the same
-// products is the same dot product), so that every lane reads D / 4 consecutive floats of its row and centroid. The
-// eight 16-centroid tiles of a 128-centroid chunk accumulate side by side (eight independent MFMA chains); centroids
-// past M are zeros in LDS and their distances are skipped.
-template <int D>
+// assign: bound by the fp32 matrix rate (B x M x D x 2 FLOP; 135 TFLOP/s in a bare loop: 49 us at 12 720 candidates x 16
+// heads x 128 clusters x 128). A wavefront keeps 32 centroids in registers for the whole pass and streams 16-candidate
+// tiles past them; the wavefronts of a block split the centroids (WR = 1: four groups of 32) or, with few of them, the
+// tiles (up to 64 clusters: WR = 2, up to 32: WR = 4). The block reads WR tiles a stage ahead in whole rows, forms x and
+// leaves it in LDS, where every wavefront finds its operands: gathered by each wavefront from memory in operand order
+// (16 bytes here and there of 32 lines per load) a pass took 85 to 97 us, and so it did with the centroids in LDS and
+// the candidates in registers.
+// MFMA 16x16x4 f32: lane l supplies A[l % 16][l / 16] (a centroid) and B[l / 16][l % 16] (a candidate) and holds
+// D[4 (l / 16) + r][l % 16]: four centroids of one candidate, so that the nearest is found in the lane but for two
+// exchanges. The reduction dimension is visited in the order d = (l / 16) * (D / 4) + s at step s (any order of the same
+// products is the same dot product), so that every lane reads D / 4 consecutive elements of its row and centroid.
+template <int D, bool BF, int WR>
+struct StageIn {
+  static constexpr int ROWS = 16 * WR;
+  static constexpr int PER = ROWS * (D / 8) / kAssignThreads > 0 ? ROWS * (D / 8) / kAssignThreads : 1;
+  u32x4 raw[PER][BF ? 1 : 2];   // 8 elements of a row per thread and step
+  float inv[PER], xx[PER];
+};
+
+__device__ __forceinline__ bool nearer(float d, int i, float od, int oi) { return d < od || (d == od && i < oi); }
+
+template <int D, bool BF, int WR>
 __global__ __launch_bounds__(kAssignThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void mem_assign_kernel(SelArgs g, int it) {
-  if (it > 0 && g.moved[it - 1] == 0) return;
-  constexpr int KS = D / 4;   // MFMA steps per dot product
-  __shared__ float cl[kCChunk * kCPitch];
-  __shared__ float ccl[kCChunk];
-  const int h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int h = blockIdx.y;
+  if (it > 0 && g.moved[(int64_t)(it - 1) * g.H + h] == 0) return;
+  typedef StageIn<D, BF, WR> Stage;
+  constexpr int KS = D / 4;          // MFMA steps per dot product
+  constexpr int WC = 4 / WR;         // centroid groups
+  constexpr int PITCH = D + 4;       // floats per row in LDS (16 rows of one 16-byte column on different banks)
+  constexpr int CPR = D / 8;         // 8-element chunks per row
+  __shared__ __attribute__((aligned(16))) float xs[2][Stage::ROWS > 32 ? Stage::ROWS : 32][PITCH];   // centroids first
+  __shared__ float xxs[2][Stage::ROWS];
+  __shared__ float bestv[WC][16 * kAssignTiles];
+  __shared__ int besti[WC][16 * kAssignTiles];
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int kq = lane >> 4, c16 = lane & 15;
-  const int b0 = blockIdx.x * kAssignRows + w * 16;
-  // A operands: candidate b0 + c16, dims kq * KS .. + KS - 1 (rows past B are zeros)
-  // every load below reads a valid row (indices clamped) and is issued before any of them is waited for; values of
-  // rows past B are then replaced by zeros
-  float a[KS];
-  {
-    const int b = b0 + c16;
-    const float keep = b < g.B ? 1.0f : 0.0f;
-    const float* xr = g.X + ((int64_t)h * g.B + min(b, g.B - 1)) * D + kq * KS;
-    f32x4v t[KS / 4];
+  const int cw = w % WC, rw = w / WC;   // this wavefront's centroid group and tile of a stage
+  const int tiles = (g.B + 15) / 16, nb = gridDim.x;
+  const int mine = ((int)blockIdx.x < tiles ? (tiles - 1 - (int)blockIdx.x) / nb : -1) + 1;   // this block's tiles
+  const int stages = (mine + WR - 1) / WR;
+  // candidate of row r of a stage (past the last: the last one again, not stored)
+  auto cand_of = [&](int stage, int r) {
+    return min(16 * ((int)blockIdx.x + nb * (WR * stage + (r >> 4))) + (r & 15), g.B - 1);
+  };
+  const bool loads = Stage::ROWS * CPR >= kAssignThreads || tid < Stage::ROWS * CPR;
+  auto load_rows = [&](int stage, int (&row)[Stage::PER]) {
 #pragma unroll
-    for (int s = 0; s < KS / 4; ++s) t[s] = *(const f32x4v*)(xr + 4 * s);
+    for (int p = 0; p < Stage::PER; ++p) {
+      const int b = cand_of(stage, (tid + p * kAssignThreads) / CPR % Stage::ROWS);
+      row[p] = BF && g.rows ? g.rows[b] : b;
+    }
+  };
+  auto load_stage = [&](int stage, const int (&row)[Stage::PER], Stage& in) {
 #pragma unroll
-    for (int s = 0; s < KS / 4; ++s)
+    for (int p = 0; p < Stage::PER; ++p) {
+      const int e = tid + p * kAssignThreads, c = e % CPR;
+      const int64_t hb = (int64_t)h * g.B + cand_of(stage, e / CPR % Stage::ROWS);
+      if constexpr (BF) {
+        in.raw[p][0] = *(const u32x4*)((const uint16_t*)g.keys + row[p] * g.stride + (int64_t)h * D + 8 * c);
+        in.inv[p] = g.inv[hb];
+      } else {
+        const u32x4* x = (const u32x4*)(g.X + hb * D + 8 * c);
+        in.raw[p][0] = x[0];
+        in.raw[p][1] = x[1];
+      }
+      in.xx[p] = g.xx[hb];
+    }
+  };
+  auto store_stage = [&](int buf, const Stage& in) {
+    if (loads)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) a[4 * s + j] = t[s][j] * keep;
-  }
-  float xxr[4];
+      for (int p = 0; p < Stage::PER; ++p) {
+        const int e = tid + p * kAssignThreads, r = e / CPR, c = e % CPR;
+        f32x4v* o = (f32x4v*)&xs[buf][r][8 * c];
+        if constexpr (BF) {
+          float x[8];
 #pragma unroll
-  for (int r = 0; r < 4; ++r) xxr[r] = g.xx[(int64_t)h * g.B + min(b0 + 4 * kq + r, g.B - 1)];
-  float best[4];
-  int besti[4];
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    best[r] = __builtin_inff();
-    besti[r] = 0;   // stays 0 only if no distance is finite (non-finite keys): still a valid cluster
-  }
+          for (int j = 0; j < 4; ++j) {
+            x[2 * j] = bf2f((uint16_t)(in.raw[p][0][j] & 0xffffu)) * in.inv[p];
+            x[2 * j + 1] = bf2f((uint16_t)(in.raw[p][0][j] >> 16)) * in.inv[p];
+          }
+          o[0] = f32x4v{x[0], x[1], x[2], x[3]};
+          o[1] = f32x4v{x[4], x[5], x[6], x[7]};
+        } else {
+          o[0] = __builtin_bit_cast(f32x4v, in.raw[p][0]);
+          o[1] = __builtin_bit_cast(f32x4v, in.raw[p][1]);
+        }
+        if (c == 0) xxs[buf][r] = in.xx[p];
+      }
+  };
   const float* Ch = g.C + (int64_t)h * g.M * D;
-  for (int c0 = 0; c0 < g.M; c0 += kCChunk) {
-    const int nc = min(kCChunk, g.M - c0);
-    __syncthreads();
-    {
-      constexpr int PER = kCChunk * (D / 4) / kAssignThreads;   // float4 per thread
-      f32x4v t[PER];
-      float ccv = 0.0f;
+  for (int c0 = 0; c0 < g.M; c0 += 32 * WC) {
+    const int ci = c0 + 32 * cw;    // this wavefront's first centroid (past the last: its results stay infinite)
+    int row[Stage::PER];
+    Stage in;
+    load_rows(0, row);
+    // the centroids by whole rows through LDS, 16 of every group at a time (group k in rows 16 k ..)
+    f32x4v cen[2][KS / 4];
+    float cc[2][4];
+    float* cs = &xs[0][0][0];
 #pragma unroll
-      for (int k = 0; k < PER; ++k) {
-        const int e = tid + k * kAssignThreads, i = e / (D / 4), d4 = e % (D / 4);
-        t[k] = *(const f32x4v*)(Ch + (int64_t)(c0 + min(i, nc - 1)) * D + 4 * d4);
+    for (int t = 0; t < 2; ++t) {
+      constexpr int N = 16 * WC * (D / 4) / kAssignThreads;   // 16-byte chunks per thread
+      f32x4v v[N];
+#pragma unroll
+      for (int n = 0; n < N; ++n) {
+        const int e = tid + n * kAssignThreads, r = e / (D / 4), i = c0 + 32 * (r >> 4) + 16 * t + (r & 15);
+        v[n] = *(const f32x4v*)(Ch + (int64_t)min(i, g.M - 1) * D + 4 * (e % (D / 4)));
       }
-      if (tid < kCChunk) ccv = g.cc[(int64_t)h * g.M + c0 + min(tid, nc - 1)];
+      __syncthreads();   // what the buffer held is no longer read
 #pragma unroll
-      for (int k = 0; k < PER; ++k) {
-        const int e = tid + k * kAssignThreads, i = e / (D / 4), d4 = e % (D / 4);
-        const float keep = i < nc ? 1.0f : 0.0f;
-        *(f32x4v*)(cl + i * kCPitch + 4 * d4) = t[k] * keep;
+      for (int n = 0; n < N; ++n) {
+        const int e = tid + n * kAssignThreads;
+        *(f32x4v*)(cs + e / (D / 4) * PITCH + 4 * (e % (D / 4))) = v[n];
       }
-      if (tid < kCChunk) ccl[tid] = tid < nc ? ccv : 0.0f;
-    }
-    __syncthreads();
-    f32x4v acc[8];
+      __syncthreads();
 #pragma unroll
-    for (int t = 0; t < 8; ++t) acc[t] = f32x4v{0.0f, 0.0f, 0.0f, 0.0f};
+      for (int s = 0; s < KS / 4; ++s) cen[t][s] = *(const f32x4v*)(cs + (16 * cw + c16) * PITCH + kq * KS + 4 * s);
 #pragma unroll
-    for (int s = 0; s < KS; s += 4) {
-#pragma unroll
-      for (int th = 0; th < 8; th += 4) {   // four tiles' operands at a time
-        f32x4v bv[4];
-#pragma unroll
-        for (int t = 0; t < 4; ++t) bv[t] = *(const f32x4v*)(cl + (16 * (th + t) + c16) * kCPitch + kq * KS + s);
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-          for (int t = 0; t < 4; ++t)
-            acc[th + t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s + j], bv[t][j], acc[th + t], 0, 0, 0);
+      for (int r = 0; r < 4; ++r) {
+        const int i = ci + 16 * t + 4 * kq + r;
+        const float v1 = g.cc[(int64_t)h * g.M + min(i, g.M - 1)];
+        cc[t][r] = i < g.M ? v1 : __builtin_inff();
       }
     }
+    load_stage(0, row, in);
+    load_rows(1, row);
+    __syncthreads();     // the centroids are in registers
+    store_stage(0, in);
+    load_stage(1, row, in);
+    load_rows(2, row);
+    for (int st = 0; st < stages; ++st) {
+      __syncthreads();   // stage st is in its buffer, and stage st - 1 no longer read
+      store_stage((st + 1) & 1, in);
+      load_stage(st + 2, row, in);
+      load_rows(st + 3, row);
+      const int n = WR * st + rw;
+      f32x4v x[KS / 4];
 #pragma unroll
-    for (int t = 0; t < 8; ++t) {
-      const int i = 16 * t + c16;
-      if (i < nc) {
-        const float cc = ccl[i];
+      for (int s = 0; s < KS / 4; ++s) x[s] = *(const f32x4v*)&xs[st & 1][16 * rw + c16][kq * KS + 4 * s];
+      const float xx = xxs[st & 1][16 * rw + c16];
+      f32x4v acc[2] = {f32x4v{0.0f, 0.0f, 0.0f, 0.0f}, f32x4v{0.0f, 0.0f, 0.0f, 0.0f}};
+#pragma unroll
+      for (int s = 0; s < KS; ++s)
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+          acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(cen[t][s / 4][s % 4], x[s / 4][s % 4], acc[t], 0, 0, 0);
+      float best = __builtin_inff();
+      int bi = 0;   // stays 0 only if no distance is finite (non-finite keys): still a valid cluster
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const float dd = (xxr[r] - 2.0f * acc[t][r]) + cc;
-          if (dd < best[r]) {    // centroids visited in ascending order: the first minimum stays
-            best[r] = dd;
-            besti[r] = c0 + i;
+          const float dd = (xx - 2.0f * acc[t][r]) + cc[t][r];
+          if (dd < best) {    // centroids visited in ascending order: the first minimum stays
+            best = dd;
+            bi = ci + 16 * t + 4 * kq + r;
           }
+        }
+#pragma unroll
+      for (int o = 16; o <= 32; o <<= 1) {
+        const float od = __shfl_xor(best, o, 64);
+        const int oi = __shfl_xor(bi, o, 64);
+        const bool nr = nearer(od, oi, best, bi);
+        best = nr ? od : best;
+        bi = nr ? oi : bi;
+      }
+      if (kq == 0 && n < mine) {   // this wavefront's own entries
+        const int e = 16 * n + c16;
+        if (c0 == 0 || nearer(best, bi, bestv[cw][e], besti[cw][e])) {
+          bestv[cw][e] = best;
+          besti[cw][e] = bi;
         }
       }
     }
   }
-  // across the 16 lanes that hold the same 4 candidates: the smallest distance, then the lowest centroid
+  __syncthreads();
+  for (int e = tid; e < 16 * mine; e += kAssignThreads) {
+    const int b = 16 * ((int)blockIdx.x + nb * (e >> 4)) + (e & 15);
+    float best = bestv[0][e];
+    int bi = besti[0][e];
 #pragma unroll
-  for (int o = 1; o < 16; o <<= 1) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const float od = __shfl_xor(best[r], o, 64);
-      const int oi = __shfl_xor(besti[r], o, 64);
-      if (od < best[r] || (od == best[r] && oi < besti[r])) {
-        best[r] = od;
-        besti[r] = oi;
+    for (int k = 1; k < WC; ++k)
+      if (nearer(bestv[k][e], besti[k][e], best, bi)) {
+        best = bestv[k][e];
+        bi = besti[k][e];
       }
-    }
-  }
-  if (c16 == 0) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int b = b0 + 4 * kq + r;
-      if (b < g.B) {
-        g.z[(int64_t)h * g.B + b] = besti[r];
-        g.dist[(int64_t)h * g.B + b] = best[r];
-      }
+    if (b < g.B) {
+      g.z[(int64_t)h * g.B + b] = bi;
+      g.dist[(int64_t)h * g.B + b] = best;
     }
   }
 }
 
 // ------------------------------------------------------------------------------------------------------------------
-// group: one workgroup of 16 wavefronts per head, a stable counting sort of the candidates by cluster. Wavefront w
-// owns the contiguous candidates [w n / 16, (w + 1) n / 16) rounded to 64; it counts them per cluster, the counts
-// are scanned cluster by cluster and, within a cluster, wavefront by wavefront, and then every wavefront places its
-// candidates in order: lanes with the same cluster find each other through ballots over the cluster's bits, so a
-// candidate's place is its wavefront's running count for the cluster plus its rank among the earlier lanes.
-__global__ __launch_bounds__(1024) void mem_group_kernel(SelArgs g, int it, int bits) {
-  // the moved flag of this iteration starts at 0 (prep set every flag to 1, so that iteration 0 always runs); the
-  // update after this kernel raises it
-  if (blockIdx.x == 0 && threadIdx.x == 0 && it < g.iters) g.moved[it] = 0;
-  if (it > 0 && g.moved[it - 1] == 0) return;
-  __shared__ int cnt[16 * kMaxClusters];   // cnt[w * M + c]
-  __shared__ int wsum[16];
-  const int h = blockIdx.x, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+// update: a block averages kUpdClusters clusters of one head, 128 threads each: four groups of 32 take the members j = q,
+// q + 4, ... (group q) in ascending order, four elements of D per thread, and the four partial sums are added in group
+// order. The block finds the members itself: it reads the head's assignments (from the L2: a few tens of KB) a chunk at a
+// time, wavefront w the w-th part of a chunk; one ballot per 64 assignments gathers the members of any of its clusters,
+// and a wavefront per cluster then picks its own from those few.
+// Bound by latency for small clusters (assignments, member rows) and by the read of the keys for many: one cluster per
+// block with four rows of 4-byte loads in flight took 28 us where the first passes put hundreds of keys into one cluster.
+template <int D, bool BF>
+__global__ __launch_bounds__(kUpdThreads) void mem_update_kernel(SelArgs g, int it) {
+  const int h = blockIdx.y;
+  if (it > 0 && g.moved[(int64_t)(it - 1) * g.H + h] == 0) return;
+  constexpr int W = kUpdThreads / 64, K = kUpdClusters;
+  __shared__ int found[kUpdChunk];      // the chunk's members of any of the clusters, cluster << 16 | place in the chunk
+  __shared__ int mrow[kUpdChunk];       // cluster after cluster, ascending: the members' key rows (fp32: candidates)
+  __shared__ float minv[kUpdChunk];
+  __shared__ int wcnt[W], beg[K], len[K];
+  __shared__ float part[K][4][128];
+  __shared__ float norm[K][128];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int i0 = blockIdx.x * K;
+  const int k = tid >> 7, q = (tid >> 5) & 3, d4 = 4 * (tid & 31);   // this thread's cluster, member group and elements
   const int32_t* zh = g.z + (int64_t)h * g.B;
-  const int per = ((g.B + 16 * 64 - 1) / (16 * 64)) * 64;
-  const int lo = min(g.B, w * per), hi = min(g.B, lo + per);
-  for (int i = tid; i < 16 * g.M; i += 1024) cnt[i] = 0;
-  __syncthreads();
-  for (int b = lo + lane; b < hi; b += 64) atomicAdd(&cnt[w * g.M + zh[b]], 1);
-  __syncthreads();
-  // per cluster c (thread c, and c + 1024 ... past 1024 clusters, which kMaxClusters excludes): its total and the
-  // exclusive prefix over the wavefronts
-  const int c = tid;
-  int tot = 0;
-  if (c < g.M)
-    for (int x = 0; x < 16; ++x) {
-      const int n = cnt[x * g.M + c];
-      cnt[x * g.M + c] = tot;
-      tot += n;
-    }
-  // exclusive scan of the totals over the clusters: within each wavefront by shuffles, then over the wavefronts
-  int incl = tot;
+  const uint64_t below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+  f32x4v sum = {0.0f, 0.0f, 0.0f, 0.0f};
+  int seen = 0;     // members of cluster k in the chunks before
+  for (int c0 = 0; c0 < g.B; c0 += kUpdChunk) {
+    int zi[kUpdPer];
 #pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int y = __shfl_up(incl, o, 64);
-    if (lane >= o) incl += y;
-  }
-  if (lane == 63) wsum[w] = incl;
-  __syncthreads();
-  int before = 0;
-  for (int x = 0; x < w; ++x) before += wsum[x];
-  const int start = before + incl - tot;
-  int32_t* st = g.start + (int64_t)h * (g.M + 1);
-  if (c < g.M) {
-    st[c] = start;
-    for (int x = 0; x < 16; ++x) cnt[x * g.M + c] += start;
-  }
-  if (c == 0) st[g.M] = g.B;
-  __syncthreads();
-  int32_t* oh = g.order + (int64_t)h * g.B;
-  const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-  int* mine = cnt + w * g.M;
-  for (int b0 = lo; b0 < hi; b0 += 64) {   // the same trip count in every lane of the wavefront
-    const int b = b0 + lane;
-    const bool in = b < hi;
-    const int cl = in ? zh[b] : -1;
-    uint64_t same = __ballot(in);
-    for (int k = 0; k < bits; ++k) {
-      const uint64_t ones = __ballot(in && ((cl >> k) & 1));
-      same &= ((cl >> k) & 1) ? ones : ~ones;
+    for (int u = 0; u < kUpdPer; ++u) {
+      const int b = c0 + w * (64 * kUpdPer) + 64 * u + lane;
+      const int z = zh[min(b, g.B - 1)];
+      zi[u] = b < g.B ? z - i0 : -1;
     }
-    const int rank = __popcll(same & below);
-    const int base = in ? mine[cl] : 0;
-    if (in) oh[base + rank] = b;
-    // every lane has read its base before the group's last lane moves the count on (one wavefront, in order)
-    __builtin_amdgcn_wave_barrier();
-    if (in && (same >> lane) == 1ull) mine[cl] = base + rank + 1;
-    __builtin_amdgcn_wave_barrier();
-  }
-}
-
-// ------------------------------------------------------------------------------------------------------------------
-// update: block (i, h) averages cluster i's members in their fixed order: four groups of 128 threads take the members
-// j = q, q + 4, ... (group q), one element of D per thread, and the four partial sums are added in group order
-__global__ __launch_bounds__(512) void mem_update_kernel(SelArgs g, int it) {
-  if (it > 0 && g.moved[it - 1] == 0) return;
-  __shared__ float part[4][128];
-  __shared__ float red[128];
-  const int i = blockIdx.x, h = blockIdx.y, d = threadIdx.x & 127, q = threadIdx.x >> 7;
-  const int32_t* st = g.start + (int64_t)h * (g.M + 1);
-  const int a = st[i], e = st[i + 1];
-  if (a == e) return;   // empty: the centroid (and its |c|^2) stays
-  const int32_t* oh = g.order + (int64_t)h * g.B;
-  const float* Xh = g.X + (int64_t)h * g.B * g.D;
-  float s = 0.0f;
-  if (d < g.D) {
-    int j = a + q;
-    for (; j + 12 < e; j += 16) {
-      const int r0 = oh[j], r1 = oh[j + 4], r2 = oh[j + 8], r3 = oh[j + 12];
-      const float x0 = Xh[(int64_t)r0 * g.D + d], x1 = Xh[(int64_t)r1 * g.D + d];
-      const float x2 = Xh[(int64_t)r2 * g.D + d], x3 = Xh[(int64_t)r3 * g.D + d];
-      s += x0;
-      s += x1;
-      s += x2;
-      s += x3;
+    int cnt = 0;
+    uint64_t bal[kUpdPer];
+#pragma unroll
+    for (int u = 0; u < kUpdPer; ++u) {
+      bal[u] = __ballot(zi[u] >= 0 && zi[u] < K);
+      cnt += __popcll(bal[u]);
     }
-    for (; j < e; j += 4) s += Xh[(int64_t)oh[j] * g.D + d];
+    if (lane == 0) wcnt[w] = cnt;
+    __syncthreads();   // the lists of the chunk before are no longer read either
+    int at = 0, all = 0;
+#pragma unroll
+    for (int x = 0; x < W; ++x) {
+      if (x < w) at += wcnt[x];
+      all += wcnt[x];
+    }
+#pragma unroll
+    for (int u = 0; u < kUpdPer; ++u) {
+      if (zi[u] >= 0 && zi[u] < K) found[at + __popcll(bal[u] & below)] = zi[u] << 16 | (w * (64 * kUpdPer) + 64 * u + lane);
+      at += __popcll(bal[u]);
+    }
+    __syncthreads();
+    if ((w & 1) == 0) {   // the first wavefront of each cluster picks its own
+      int before = 0, n = 0;
+      for (int x = 0; x < all; x += 64) before += __popcll(__ballot(x + lane < all && found[x + lane] >> 16 < k));
+      for (int x = 0; x < all; x += 64) {
+        const int f = x + lane < all ? found[x + lane] : -1;
+        const uint64_t own = __ballot(f >> 16 == k);
+        if (f >> 16 == k) {
+          const int place = before + n + __popcll(own & below), b = c0 + (f & 0xffff);
+          mrow[place] = BF && g.rows ? g.rows[b] : b;
+          if constexpr (BF) minv[place] = g.inv[(int64_t)h * g.B + b];
+        }
+        n += __popcll(own);
+      }
+      if (lane == 0) {
+        beg[k] = before;
+        len[k] = n;
+      }
+    }
+    __syncthreads();
+    const int n = len[k], mine = beg[k];
+    if (d4 < D) {
+      for (int m = (q - seen) & 3; m < n; m += 4 * kUpdFly) {
+        f32x4v x[kUpdFly];
+#pragma unroll
+        for (int u = 0; u < kUpdFly; ++u) {
+          const int j = mine + min(m + 4 * u, n - 1);
+          if constexpr (BF) {
+#pragma clang fp contract(off)
+            const uint2 v = *(const uint2*)((const uint16_t*)g.keys + mrow[j] * g.stride + (int64_t)h * D + d4);
+            const float inv = minv[j];
+            x[u] = f32x4v{bf2f((uint16_t)(v.x & 0xffffu)) * inv, bf2f((uint16_t)(v.x >> 16)) * inv,
+                          bf2f((uint16_t)(v.y & 0xffffu)) * inv, bf2f((uint16_t)(v.y >> 16)) * inv};
+          } else {
+            x[u] = *(const f32x4v*)(g.X + ((int64_t)h * g.B + mrow[j]) * D + d4);
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < kUpdFly; ++u)
+          if (m + 4 * u < n)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+#pragma clang fp contract(off)
+              sum[e] = sum[e] + x[u][e];
+            }
+      }
+    }
+    seen += n;
   }
-  part[q][d] = s;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) part[k][q][d4 + e] = sum[e];
   __syncthreads();
+  const int d = tid & 127, i = i0 + k;
+  const bool live = i < g.M && seen > 0;   // empty: the centroid (and its |c|^2) stays
   float c = 0.0f;
   bool change = false;
-  if (q == 0 && d < g.D) {
-    c = ((part[0][d] + part[1][d]) + part[2][d]) + part[3][d];
-    c = c / (float)(e - a);
-    float* cp = g.C + ((int64_t)h * g.M + i) * g.D + d;
+  if (live && d < D) {
+    c = ((part[k][0][d] + part[k][1][d]) + part[k][2][d]) + part[k][3][d];
+    c = c / (float)seen;
+    float* cp = g.C + ((int64_t)h * g.M + i) * D + d;
     change = *cp != c;
     *cp = c;
   }
-  // |c|^2 by the fixed tree (every thread takes part in the barriers; group 0 holds the values)
-  const float n2 = centroid_norm2(q == 0 ? c : 0.0f, q == 0 ? d : 128, g.D, red);
-  if (threadIdx.x == 0) g.cc[(int64_t)h * g.M + i] = n2;
-  if (__syncthreads_or(change) && threadIdx.x == 0) atomicOr(&g.moved[it], 1);
+  // |c|^2 by the tree of centroid_norm2: the halves of the row first, then within a wavefront
+  norm[k][d] = c * c;
+  const bool any = __syncthreads_or(change);
+  if (d < 64) {
+    float n2 = norm[k][d] + norm[k][d + 64];
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) n2 += __shfl_down(n2, o, 64);
+    if (d == 0 && live) g.cc[(int64_t)h * g.M + i] = n2;
+  }
+  if (any && tid == 0) atomicOr(&g.moved[(int64_t)it * g.H + h], 1);
 }
 
 // ------------------------------------------------------------------------------------------------------------------
-// medoid: one workgroup per head; wavefront w takes clusters w, w + 16, ...; rep / valid compacted in cluster order
+// medoid: one workgroup per head. The smallest (distance, candidate) of every cluster by 64-bit minima in LDS (the
+// distance's bits mapped so that their order is that of the values); rep / valid compacted in cluster order.
 __global__ __launch_bounds__(1024) void mem_medoid_kernel(SelArgs g) {
-  __shared__ int pick[kMaxClusters];
-  __shared__ int slot[kMaxClusters];
-  const int h = blockIdx.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int32_t* st = g.start + (int64_t)h * (g.M + 1);
-  const int32_t* oh = g.order + (int64_t)h * g.B;
+  __shared__ unsigned long long pick[kMaxClusters];
+  __shared__ int wsum[16];
+  const int h = blockIdx.x, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int32_t* zh = g.z + (int64_t)h * g.B;
   const float* dh = g.dist + (int64_t)h * g.B;
-  for (int i = w; i < g.M; i += 16) {
-    const int a = st[i], e = st[i + 1];
-    float bd = __builtin_inff();
-    int bb = 0x7fffffff;
-    for (int j = a + lane; j < e; j += 64) {
-      const int b = oh[j];
-      const float dd = dh[b];
-      if (dd < bd || (dd == bd && b < bb)) {
-        bd = dd;
-        bb = b;
-      }
+  pick[tid] = ~0ull;
+  __syncthreads();
+  for (int b0 = tid; b0 < g.B; b0 += 4 * 1024) {
+    int z[4];
+    float d[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int b = min(b0 + 1024 * u, g.B - 1);   // the last candidate again: no change
+      z[u] = zh[b];
+      d[u] = dh[b];
     }
 #pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) {
-      const float od = __shfl_xor(bd, o, 64);
-      const int ob = __shfl_xor(bb, o, 64);
-      if (od < bd || (od == bd && ob < bb)) {
-        bd = od;
-        bb = ob;
-      }
+    for (int u = 0; u < 4; ++u) {
+      const uint32_t x = __float_as_uint(d[u] + 0.0f);   // -0 equals +0
+      const uint32_t ord = x & 0x80000000u ? ~x : x | 0x80000000u;
+      const unsigned long long key = (unsigned long long)ord << 32 | (uint32_t)min(b0 + 1024 * u, g.B - 1);
+      if (key < pick[z[u]]) atomicMin(&pick[z[u]], key);
     }
-    if (lane == 0) pick[i] = a < e ? bb : -1;
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    int r = 0;
-    for (int i = 0; i < g.M; ++i) slot[i] = pick[i] >= 0 ? r++ : -1;
-  }
+  const bool has = tid < g.M && pick[tid] != ~0ull;
+  const uint64_t bal = __ballot(has);
+  if (lane == 0) wsum[w] = __popcll(bal);
   __syncthreads();
+  int before = 0, total = 0;
+#pragma unroll
+  for (int x = 0; x < 16; ++x) {
+    if (x < w) before += wsum[x];
+    total += wsum[x];
+  }
   int64_t* rp = g.rep + (int64_t)h * g.M;
   uint8_t* vp = g.valid + (int64_t)h * g.M;
-  for (int i = threadIdx.x; i < g.M; i += 1024) {
-    rp[i] = 0;
-    vp[i] = 0;
+  if (has) {
+    const int r = before + __popcll(bal & (lane == 0 ? 0ull : (~0ull >> (64 - lane))));
+    rp[r] = (int64_t)(pick[tid] & 0xffffffffull);
+    vp[r] = 1;
   }
-  __syncthreads();
-  for (int i = threadIdx.x; i < g.M; i += 1024)
-    if (slot[i] >= 0) {
-      rp[slot[i]] = pick[i];
-      vp[slot[i]] = 1;
-    }
+  if (tid >= total && tid < g.M) {
+    rp[tid] = 0;
+    vp[tid] = 0;
+  }
 }
 
 // ------------------------------------------------------------------------------------------------------------------
@@ -521,8 +620,13 @@ __global__ __launch_bounds__(256) void mem_foreign_kernel(const int64_t* rep, co
   if (tid == 0) k_len_head[(int64_t)i * H + h] = piece_len[i] + total;
 }
 
+template <int D, bool BF>
+auto assign_fn(int share) {
+  return share == 4 ? mem_assign_kernel<D, BF, 4> : share == 2 ? mem_assign_kernel<D, BF, 2> : mem_assign_kernel<D, BF, 1>;
+}
+
 struct WsParts {
-  int64_t X, xx, cc, z, dist, order, start, moved, total;
+  int64_t X, inv, xx, cc, z, dist, moved, total;
 };
 
 WsParts ws_parts(int B, int H, int D, int M, int iters) {
@@ -534,13 +638,12 @@ WsParts ws_parts(int B, int H, int D, int M, int iters) {
     return at;
   };
   p.X = take((int64_t)H * B * D * 4);
+  p.inv = take((int64_t)H * B * 4);
   p.xx = take((int64_t)H * B * 4);
   p.cc = take((int64_t)H * M * 4);
   p.z = take((int64_t)H * B * 4);
   p.dist = take((int64_t)H * B * 4);
-  p.order = take((int64_t)H * B * 4);
-  p.start = take((int64_t)H * (M + 1) * 4);
-  p.moved = take((int64_t)(iters + 1) * 4);
+  p.moved = take((int64_t)(iters + 1) * H * 4);
   p.total = o;
   return p;
 }
@@ -584,30 +687,34 @@ extern "C" int or_memory_select(const void* keys, int32_t fp32_keys, const int32
   g.fp32_in = fp32_keys ? 1 : 0;
   g.iters = iters;
   g.X = (float*)(w + wp.X);
+  g.inv = (float*)(w + wp.inv);
   g.xx = (float*)(w + wp.xx);
   g.cc = (float*)(w + wp.cc);
   g.C = centroids;
   g.z = (int32_t*)(w + wp.z);
   g.dist = (float*)(w + wp.dist);
-  g.order = (int32_t*)(w + wp.order);
-  g.start = (int32_t*)(w + wp.start);
   g.moved = (int32_t*)(w + wp.moved);
   g.rep = rep;
   g.valid = valid;
   hipStream_t st = (hipStream_t)stream;
-  if (D == 128) hipLaunchKernelGGL(mem_prep_kernel<128>, dim3((B + 3) / 4, (H + 15) / 16), dim3(256), 0, st, g, iters + 1);
-  else hipLaunchKernelGGL(mem_prep_kernel<64>, dim3((B + 3) / 4, (H + 31) / 32), dim3(256), 0, st, g, iters + 1);
+  const int n_moved = (iters + 1) * H;
+  if (D == 128) hipLaunchKernelGGL(mem_prep_kernel<128>, dim3((B + 3) / 4, (H + 15) / 16), dim3(256), 0, st, g, n_moved);
+  else hipLaunchKernelGGL(mem_prep_kernel<64>, dim3((B + 3) / 4, (H + 31) / 32), dim3(256), 0, st, g, n_moved);
   if (int rc = check_hip(hipGetLastError(), "mem_prep_kernel launch")) return rc;
   hipLaunchKernelGGL(mem_start_kernel, dim3(M, H), dim3(128), 0, st, g, init);
   if (int rc = check_hip(hipGetLastError(), "mem_start_kernel launch")) return rc;
-  int bits = 0;
-  while ((1 << bits) < M) ++bits;
-  const dim3 agrid((B + kAssignRows - 1) / kAssignRows, H);
+  // the tiles of a head over enough blocks to fill the chip twice
+  const int share = M <= 32 ? 4 : M <= 64 ? 2 : 1, tiles = (B + 15) / 16;
+  const int nb = std::max(std::min((tiles + share - 1) / share, std::max(1, kPassBlocks / H)),
+                          (tiles + kAssignTiles - 1) / kAssignTiles);
+  const dim3 agrid(nb, H), ugrid((M + kUpdClusters - 1) / kUpdClusters, H);
+  const auto assign = D == 128 ? (fp32_keys ? assign_fn<128, false>(share) : assign_fn<128, true>(share))
+                               : (fp32_keys ? assign_fn<64, false>(share) : assign_fn<64, true>(share));
+  const auto update = D == 128 ? (fp32_keys ? mem_update_kernel<128, false> : mem_update_kernel<128, true>)
+                               : (fp32_keys ? mem_update_kernel<64, false> : mem_update_kernel<64, true>);
   for (int it = 0; it <= iters; ++it) {
-    if (D == 128) hipLaunchKernelGGL(mem_assign_kernel<128>, agrid, dim3(kAssignThreads), 0, st, g, it);
-    else hipLaunchKernelGGL(mem_assign_kernel<64>, agrid, dim3(kAssignThreads), 0, st, g, it);
-    hipLaunchKernelGGL(mem_group_kernel, dim3(H), dim3(1024), 0, st, g, it, bits);
-    if (it < iters) hipLaunchKernelGGL(mem_update_kernel, dim3(M, H), dim3(512), 0, st, g, it);
+    hipLaunchKernelGGL(assign, agrid, dim3(kAssignThreads), 0, st, g, it);
+    if (it < iters) hipLaunchKernelGGL(update, ugrid, dim3(kUpdThreads), 0, st, g, it);
     if (int rc = check_hip(hipGetLastError(), "k-means launch")) return rc;
   }
   hipLaunchKernelGGL(mem_medoid_kernel, dim3(H), dim3(1024), 0, st, g);
