@@ -369,6 +369,18 @@ int or_memory_foreign(const int64_t* rep, const uint8_t* valid, const int64_t* c
                       const int32_t* k_off, int32_t n_pieces, int32_t H, int32_t M, int32_t* fsrc, int32_t* fdst,
                       int32_t* k_len_head, void* stream);
 
+/* n int32 values of host memory into device memory by kernel launches that carry them (896 each): no copy, and the host
+ * array is free on return. */
+int or_index_fill(const int32_t* values, int32_t n, int32_t* out, void* stream);
+
+/* The concatenations and offsets of attention.packed (src/onereel/attention.py:56-71): n_seg sequences of nq[s] query and
+ * nk[s] key and value rows (q, k, v: host arrays of device pointers; contiguous rows of row_bytes, a multiple of 16,
+ * 16-byte aligned) end to end into q_out, k_out and v_out, and [0, cumsum] of nq and nk into cu_q and cu_k (int32
+ * [n_seg + 1], device). One launch per 112 sequences. */
+int or_concat(const void* const* q, const void* const* k, const void* const* v, const int32_t* nq, const int32_t* nk,
+              int32_t n_seg, int64_t row_bytes, void* q_out, void* k_out, void* v_out, int32_t* cu_q, int32_t* cu_k,
+              void* stream);
+
 /* Message of the calling thread's last failed call ("" if none). */
 const char* or_last_error(void);
 

@@ -88,6 +88,8 @@ SIGNATURES = {
     'or_memory_select': (i32, [vp, i32, vp, i64, i32, i32, i32, i32, vp, vp, i32, vp, vp, vp, i64, vp]),
     'or_memory_index': (i32, [vp, vp, vp, vp, vp, vp, vp, vp, i32, i32, i32, vp, vp, vp]),
     'or_memory_foreign': (i32, [vp, vp, vp, vp, vp, vp, vp, vp, i32, i32, i32, vp, vp, vp, vp]),
+    'or_index_fill': (i32, [vp, i32, vp, vp]),
+    'or_concat': (i32, [vp, vp, vp, vp, vp, i32, i64, vp, vp, vp, vp, vp, vp]),
     'or_last_error': (ctypes.c_char_p, []),
     'or_version': (ctypes.c_char_p, []),
 }
@@ -193,6 +195,20 @@ def bench_check(rc: int, what: str):
 def ptr(t):
     """device pointer of a tensor, or None"""
     return None if t is None else t.data_ptr()
+
+
+def device_ints(lists, device):
+    """lists of Python ints as int32 tensors on the device: parts of one tensor, filled by launches that carry the
+    values (a copy from pageable memory would cost each list about 10 us of the host's time)"""
+    device = torch.device(device)
+    flat = [int(x) for values in lists for x in values]
+    if device.type != 'cuda' or not flat or min(flat) < -2 ** 31 or max(flat) >= 2 ** 31:
+        return [torch.tensor(list(values), dtype=torch.int32, device=device) for values in lists]
+    out = torch.empty(len(flat), dtype=torch.int32, device=device)
+    with torch.cuda.device(out.device):
+        check(lib().or_index_fill((ctypes.c_int32 * len(flat))(*flat), len(flat), out.data_ptr(),
+                                  stream_handle(out.device)), 'or_index_fill')
+    return list(out.split([len(values) for values in lists]))
 
 
 def stream_handle(device=None):

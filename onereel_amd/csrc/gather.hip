@@ -11,6 +11,10 @@
 // cached stores for the pack and the scatter). The rotation is done in
 // fp32 as two rounded products and a rounded sum per element (no fused multiply-add), then rounded to bf16 to
 // nearest even: the same bits as torch's x.float() * cos + rot(x).float() * sin followed by .to(bfloat16).
+#include <string.h>
+
+#include <algorithm>
+
 #include "common.h"
 
 namespace onereel {
@@ -300,6 +304,63 @@ int shared_d0(int H, int D) {
   return (8 * cp) % D == 0 ? 1 : 0;
 }
 
+// ------------------------------------------------------------------------------------------------------------------
+// Host integers to the device with the launch itself: a copy of a few offsets from pageable memory costs the host about
+// 10 us each and the GPU 2 to 4 (a Wan cross-attention call made three of them), a launch that carries them 2 to 3 us
+// for all. kFillInts: what fits the 4 KB of kernel arguments.
+constexpr int kFillInts = 896;
+struct FillArgs {
+  int32_t v[kFillInts];
+};
+
+__global__ __launch_bounds__(kThreads) void index_fill_kernel(FillArgs g, int n, int32_t* out) {
+  const int i = blockIdx.x * kThreads + threadIdx.x;
+  if (i < n) out[i] = g.v[i];
+}
+
+// The rows of up to kCatSegs q, k and v tensors end to end, and the two offset arrays of a varlen call, in one launch
+// (three concatenations and two copies of offsets before it: 44 us of GPU time for 12 sequences of 3111 query and 3638
+// key rows x 16 heads x 128, now 15). HBM-bound (every byte read and written once): a block writes 16-byte chunks of one of the
+// three results, each thread finding its chunk's sequence among the offsets in LDS; eight chunks in flight per thread.
+constexpr int kCatSegs = 112;
+constexpr int kCatFly = 8;
+struct CatArgs {
+  const u32x4* src[3][kCatSegs];
+  int32_t q_at[kCatSegs + 1], k_at[kCatSegs + 1];   // rows before each sequence in the results (from the call's first)
+};
+
+__global__ __launch_bounds__(kThreads) void concat_kernel(CatArgs g, int n_seg, int chunks, u32x4* q, u32x4* k, u32x4* v,
+                                                          int32_t* cu_q, int32_t* cu_k) {
+  __shared__ int at[kCatSegs + 1];
+  __shared__ const u32x4* src[kCatSegs];
+  const int which = blockIdx.y;
+  for (int s = threadIdx.x; s <= n_seg; s += kThreads) {
+    at[s] = which ? g.k_at[s] : g.q_at[s];
+    if (s < n_seg) src[s] = g.src[which][s];
+    if (blockIdx.x == 0 && which < 2) (which ? cu_k : cu_q)[s] = at[s];
+  }
+  __syncthreads();
+  u32x4* out = which == 0 ? q : which == 1 ? k : v;
+  const int64_t lo = (int64_t)at[0] * chunks, hi = (int64_t)at[n_seg] * chunks, per = kThreads * kCatFly;
+  for (int64_t c0 = lo + blockIdx.x * per + threadIdx.x; c0 < hi; c0 += gridDim.x * per) {
+    u32x4 x[kCatFly];
+#pragma unroll
+    for (int u = 0; u < kCatFly; ++u) {
+      const int64_t c = min(c0 + u * kThreads, hi - 1);
+      int a = 0, b = n_seg - 1;   // the last sequence that starts at or before c (empty ones before it are passed by)
+      while (a < b) {
+        const int m = (a + b + 1) >> 1;
+        if ((int64_t)at[m] * chunks <= c) a = m;
+        else b = m - 1;
+      }
+      x[u] = src[a][c - (int64_t)at[a] * chunks];
+    }
+#pragma unroll
+    for (int u = 0; u < kCatFly; ++u)
+      if (c0 + u * kThreads < hi) out[c0 + u * kThreads] = x[u];
+  }
+}
+
 }  // namespace
 }  // namespace onereel
 
@@ -470,4 +531,60 @@ extern "C" int or_scatter(const void* packed, const int32_t* dst_idx, int64_t n_
                        (hipStream_t)stream, g);
   }
   return check_hip(hipGetLastError(), "scatter_kernel launch");
+}
+
+extern "C" int or_index_fill(const int32_t* values, int32_t n, int32_t* out, void* stream) {
+  if (n < 0 || (n > 0 && (!values || !out))) return fail_arg("or_index_fill: need n >= 0, values and out");
+  for (int at = 0; at < n; at += kFillInts) {
+    const int m = std::min(kFillInts, n - at);
+    FillArgs g;
+    memcpy(g.v, values + at, (size_t)m * 4);
+    memset(g.v + m, 0, (size_t)(kFillInts - m) * 4);
+    hipLaunchKernelGGL(index_fill_kernel, dim3((m + kThreads - 1) / kThreads), dim3(kThreads), 0, (hipStream_t)stream, g,
+                       m, out + at);
+    if (int rc = check_hip(hipGetLastError(), "index_fill_kernel launch")) return rc;
+  }
+  return 0;
+}
+
+extern "C" int or_concat(const void* const* q, const void* const* k, const void* const* v, const int32_t* nq,
+                         const int32_t* nk, int32_t n_seg, int64_t row_bytes, void* q_out, void* k_out, void* v_out,
+                         int32_t* cu_q, int32_t* cu_k, void* stream) {
+  if (n_seg < 1 || row_bytes < 16 || row_bytes % 16 || row_bytes > (1 << 24))
+    return fail_arg("or_concat: need n_seg >= 1 and rows of a multiple of 16 bytes (n_seg=%d row_bytes=%lld)", n_seg,
+                    (long long)row_bytes);
+  if (!q || !k || !v || !nq || !nk || !q_out || !k_out || !v_out || !cu_q || !cu_k)
+    return fail_arg("or_concat: every array is required");
+  if (((uintptr_t)q_out | (uintptr_t)k_out | (uintptr_t)v_out) & 15u)
+    return fail_arg("or_concat: the results must be 16-byte aligned");
+  int64_t tq = 0, tk = 0;
+  for (int s = 0; s < n_seg; ++s) {
+    if (nq[s] < 0 || nk[s] < 0 || (tq += nq[s]) > 0x7fffffff || (tk += nk[s]) > 0x7fffffff)
+      return fail_arg("or_concat: row counts must be >= 0 and add up to less than 2^31");
+    if ((nq[s] && !q[s]) || (nk[s] && (!k[s] || !v[s])) || (((uintptr_t)q[s] | (uintptr_t)k[s] | (uintptr_t)v[s]) & 15u))
+      return fail_arg("or_concat: sequence %d: 16-byte aligned rows are required", s);
+  }
+  const int chunks = (int)(row_bytes / 16);
+  int64_t q0 = 0, k0 = 0;
+  for (int at = 0; at < n_seg; at += kCatSegs) {
+    const int m = std::min(kCatSegs, n_seg - at);
+    CatArgs g;
+    memset(&g, 0, sizeof(g));
+    g.q_at[0] = (int32_t)q0;
+    g.k_at[0] = (int32_t)k0;
+    for (int s = 0; s < m; ++s) {
+      g.src[0][s] = (const u32x4*)q[at + s];
+      g.src[1][s] = (const u32x4*)k[at + s];
+      g.src[2][s] = (const u32x4*)v[at + s];
+      g.q_at[s + 1] = (int32_t)(q0 += nq[at + s]);
+      g.k_at[s + 1] = (int32_t)(k0 += nk[at + s]);
+    }
+    const int64_t most = (int64_t)std::max(g.q_at[m] - g.q_at[0], g.k_at[m] - g.k_at[0]) * chunks;
+    const int64_t blocks = std::min<int64_t>(std::max<int64_t>((most + kThreads * kCatFly - 1) / (kThreads * kCatFly), 1),
+                                             4096);
+    hipLaunchKernelGGL(concat_kernel, dim3((unsigned)blocks, 3), dim3(kThreads), 0, (hipStream_t)stream, g, m, chunks,
+                       (u32x4*)q_out, (u32x4*)k_out, (u32x4*)v_out, cu_q + at, cu_k + at);
+    if (int rc = check_hip(hipGetLastError(), "concat_kernel launch")) return rc;
+  }
+  return 0;
 }
