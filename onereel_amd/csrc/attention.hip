@@ -14,7 +14,7 @@
 // - K and V stream in blocks of 32 keys through rings of LDS slots, filled by LDS DMA (buffer_load ... lds) several
 //   blocks ahead; rows past a segment's end read as zeros.
 // - head_dim 128: attn8_kernel, 64 queries per wavefront (one wavefront per SIMD), O in AGPRs, key loop in generated
-//   asm. head_dim 64: attn4_kernel, 32 queries per wavefront, two wavefronts per SIMD.
+//   asm. head_dim 64: attn4_kernel, 32 queries per wavefront, three wavefronts per SIMD.
 // - head_dim 128 with at most 256 keys per segment: attn_short_kernel, keys and values of a segment-head in LDS for the
 //   whole item, no planner and no queues.
 // - Softmax in base 2, p = 2^(c (s - m)) with c = scale * log2(e), and a running max m raised only when needed.
@@ -551,7 +551,11 @@ __device__ __forceinline__ float pair_sum(float x) {
 // 32 keys. K and V blocks stream through two rings of four LDS slots each, filled by buffer loads straight into LDS (LDS DMA) three iterations ahead; rows past a
 // segment's end read as zeros. Iteration j of a wavefront runs the softmax of block j on the VALU while the MFMA unit
 // computes S of block j + 1 (QK^T) and O += V P^T of block j - 1, so the exponentials overlap the matrix work inside
-// one wavefront as well as across the two wavefronts that share a SIMD.
+// one wavefront as well as across the wavefronts that share a SIMD. At head_dim 64 the vector work (55 instructions, 16 of
+// them exponentials, per 8 MFMAs) is longer than the matrix work, and a wavefront also waits for its LDS reads and its
+// block's barrier: a third wavefront per SIMD (145 registers, 33 KB of LDS per block; a fourth would spill) fills those
+// waits: 4 x 8192 x 8192 x 16 heads 929 -> 990 TFLOP/s, 2 x 3001 x 3001 x 16 (768 blocks in one round instead of 1.5)
+// 100 -> 89 us for the kernel, 1 x 8192 x 8192 x 12 426 -> 232 us for the call.
 //
 // Running max: P(j) is computed with the running max m as it stands; only when some probability of the block
 // exceeds 2^16 (its row-half sum exceeds 2^20, or overflows) does the wavefront take the max of the block, rescale O
@@ -779,7 +783,7 @@ __device__ __forceinline__ void iter4(St4<D>& st, const Ring& rg, int j, int nb,
 }
 
 template <int D>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3, 3)))
 void attn4_kernel(AttnArgs a, int32_t* ws) {
   using C = R4<D>;
   constexpr int WQ = 32, BQ = 4 * WQ;
