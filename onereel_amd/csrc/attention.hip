@@ -96,6 +96,12 @@ struct AttnArgs {
   int64_t n_ktok;
   // value events of the segments with value runs (kVEvents int4 per segment, written by the planner)
   const int4* v_events;
+  // what a block that finds its item itself reads besides (per segment; k_len_head per segment and head)
+  const int32_t* v_row;
+  const int32_t* v_lead;
+  const int32_t* k_lead;
+  const int32_t* k_len_head;
+  int32_t n_seg;
 };
 
 // the list a work item without further value events points its key loop at: sentinels only
@@ -782,7 +788,37 @@ __device__ __forceinline__ void iter4(St4<D>& st, const Ring& rg, int j, int nb,
   st.lsum += ls;
 }
 
-template <int D>
+// the segment of tile `tile` of the segments' tiles of `rows` queries in order, and its tile within the segment (-1: past
+// the last tile); every lane of a wavefront calls it, 64 segments looked at at a time
+__device__ __forceinline__ int tile_segment(const int32_t* cu_q, int n_seg, int rows, int lane, int& tile) {
+  int seg = -1;
+  for (int s0 = 0; s0 < n_seg; s0 += 64) {
+    const int s = s0 + lane;
+    const int lq = s < n_seg ? cu_q[s + 1] - cu_q[s] : 0;
+    int incl = lq > 0 ? (lq + rows - 1) / rows : 0;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int y = __shfl_up(incl, o, 64);
+      if (lane >= o) incl += y;
+    }
+    const int total = __shfl(incl, 63, 64);
+    if (tile < total) {
+      const int before = __popcll(__ballot(incl <= tile));   // incl does not decrease: the lanes below
+      seg = s0 + before;
+      if (before > 0) tile -= __shfl(incl, before - 1, 64);
+      break;
+    }
+    tile -= total;
+  }
+  tile = __builtin_amdgcn_readfirstlane(tile);
+  return __builtin_amdgcn_readfirstlane(seg);
+}
+
+// DIRECT: block b is the b-th (tile, head) of the call and finds its item itself, as the planner would have written it:
+// calls whose items all fit the chip at once need no order and no queues. Without the planner's launch the layer of 2
+// scenes x 3 frames x 64 tokens x 2 heads takes 35 us instead of 38 (its kernels 14 instead of 24; the rest is the host),
+// 2 x 3001 x 3001 x 16 heads 85 instead of 93.
+template <int D, bool DIRECT>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3, 3)))
 void attn4_kernel(AttnArgs a, int32_t* ws) {
   using C = R4<D>;
@@ -821,17 +857,32 @@ void attn4_kernel(AttnArgs a, int32_t* ws) {
   }
 
   const int xcc = xcc_id();
-  load_queues(ws, &qinfo, tid);
-  __syncthreads();
+  if constexpr (!DIRECT) {
+    load_queues(ws, &qinfo, tid);
+    __syncthreads();
+  }
   for (;;) {
-    if (tid == 0) item_sh = next_item(ws, xcc, &qinfo);
-    __syncthreads();
-    const int it = __builtin_amdgcn_readfirstlane(item_sh);
-    __syncthreads();
-    if (it < 0) break;
-    const int4 r0 = *(const int4*)(ws + kWsHeader + kItemWords * it);
-    const int4 r1 = *(const int4*)(ws + kWsHeader + kItemWords * it + 4);
-    const int4 r2 = *(const int4*)(ws + kWsHeader + kItemWords * it + 8);
+    int4 r0, r1, r2;
+    if constexpr (DIRECT) {
+      int tile = blockIdx.x / a.H;
+      const int hd = blockIdx.x % a.H, s = tile_segment(a.cu_q, a.n_seg, BQ, lane, tile);
+      if (s < 0) break;   // the grid covers the most tiles the call can have
+      const int qb = a.cu_q[s], ka = a.k_off ? a.k_off[s] : a.cu_k[s];
+      int lk = a.k_len ? a.k_len[s] : a.cu_k[s + 1] - a.cu_k[s];
+      if (a.k_len_head) lk = min(a.k_len_head[(int64_t)s * a.H + hd], lk);
+      r0 = make_int4((tile << 8) | hd, 0, 0, qb);
+      r1 = make_int4(a.cu_q[s + 1] - qb, a.seg_q_src ? a.seg_q_src[s] : qb, ka, lk < 0 ? 0 : lk);
+      r2 = make_int4(a.v_row ? a.v_row[s] : 0, a.v_lead ? a.v_lead[s] : 0, a.k_lead ? a.k_lead[s] : 0, -1);
+    } else {
+      if (tid == 0) item_sh = next_item(ws, xcc, &qinfo);
+      __syncthreads();
+      const int it = __builtin_amdgcn_readfirstlane(item_sh);
+      __syncthreads();
+      if (it < 0) break;
+      r0 = *(const int4*)(ws + kWsHeader + kItemWords * it);
+      r1 = *(const int4*)(ws + kWsHeader + kItemWords * it + 4);
+      r2 = *(const int4*)(ws + kWsHeader + kItemWords * it + 8);
+    }
     const int head = r0.x & 255, qt = r0.x >> 8;
     const int q_beg = r0.w, Lq = r1.x, q_src0 = r1.y, k_beg = r1.z, Lk = r1.w;
     const int q0 = qt * BQ + w * WQ;
@@ -933,6 +984,7 @@ void attn4_kernel(AttnArgs a, int32_t* ws) {
           a.lse[(int64_t)head * a.sum_q + q_beg + i] = nb > 0 ? st.m * a.scale + logf(ltot) : -__builtin_inff();
       }
     }
+    if constexpr (DIRECT) break;
   }
 }
 
@@ -1407,27 +1459,8 @@ void attn_short_kernel(AttnArgs a, int n_seg, int item_rows) {
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, h = lane >> 5;
   // this block's item: tile `tile` (item_rows queries) of the segments' tiles in order, and a head
-  int tile = blockIdx.x / a.H, seg = -1;
-  for (int s0 = 0; s0 < n_seg; s0 += 64) {
-    const int s = s0 + lane;
-    const int lq = s < n_seg ? a.cu_q[s + 1] - a.cu_q[s] : 0;
-    int incl = lq > 0 ? (lq + item_rows - 1) / item_rows : 0;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int y = __shfl_up(incl, o, 64);
-      if (lane >= o) incl += y;
-    }
-    const int total = __shfl(incl, 63, 64);
-    if (tile < total) {
-      const int before = __popcll(__ballot(incl <= tile));   // incl does not decrease: the lanes below
-      seg = s0 + before;
-      if (before > 0) tile -= __shfl(incl, before - 1, 64);
-      break;
-    }
-    tile -= total;
-  }
-  seg = __builtin_amdgcn_readfirstlane(seg);
-  tile = __builtin_amdgcn_readfirstlane(tile);
+  int tile = blockIdx.x / a.H;
+  const int seg = tile_segment(a.cu_q, n_seg, item_rows, lane, tile);
   if (seg < 0) return;   // the grid covers the most tiles the call can have
   ShortItem x;
   x.head = blockIdx.x % a.H;
@@ -1516,7 +1549,7 @@ void attn_short_kernel(AttnArgs a, int n_seg, int item_rows) {
 typedef void (*AttnFn)(AttnArgs, int32_t*);
 
 // head_dim 128 runs the 64-query kernel (256-query items), head_dim 64 the 32-query kernel (128-query items)
-AttnFn attn_fn(int D) { return D == 128 ? attn8_kernel : attn4_kernel<64>; }
+AttnFn attn_fn(int D) { return D == 128 ? attn8_kernel : attn4_kernel<64, false>; }
 int item_bq(int D) { return D == 128 ? 256 : 128; }
 
 struct DevInfo {
@@ -1706,6 +1739,20 @@ int launch_varlen(const or_varlen_args& x, void* wsp, int64_t cap, hipStream_t s
   a.split_lse = (float*)((char*)wsp + wl.lse);
   a.split_o = (float*)((char*)wsp + wl.o);
   a.v_events = (const int4*)((char*)wsp + wl.ev);
+  a.v_row = x.v_tok || x.k_tok ? x.v_row : nullptr;
+  a.v_lead = x.v_tok ? x.v_lead : nullptr;
+  a.k_lead = x.k_tok ? x.k_lead : nullptr;
+  a.k_len_head = x.k_len_head;
+  a.n_seg = x.n_seg;
+  // at head_dim 64, a call whose items are resident all at once (n segments of sum_q queries together have at most
+  // (sum_q + (b - 1) n) / b tiles of b queries) runs without the planner; with more, the planner's order (longest
+  // segments first, XCD by XCD) is worth its launch. Up to 256 segments, as attn_short_kernel.
+  const int bq = item_bq(x.D);
+  const int64_t most = (x.sum_q + (int64_t)(bq - 1) * x.n_seg) / bq * x.H;
+  if (x.D == 64 && x.n_seg <= kShortSegs && most <= grid_slots(di, x.D)) {
+    hipLaunchKernelGGL((attn4_kernel<64, true>), dim3((unsigned)most), dim3(kThreads), 0, st, a, ws);
+    return check_hip(hipGetLastError(), "attn4_kernel launch");
+  }
   VRunArgs vra;
   vra.runs = x.v_tok ? x.v_runs : nullptr;
   vra.v_tok = (uint64_t)x.v_tok;
