@@ -212,4 +212,9 @@ def device_ints(lists, device):
 
 
 def stream_handle(device=None):
-    return torch.cuda.current_stream(device).cuda_stream
+    """the current stream of the device (default: the current one), as a handle. The Stream object that
+    torch.cuda.current_stream makes for it costs more than a launch's arguments."""
+    index = device.index if isinstance(device, torch.device) else device
+    if index is None:
+        index = torch.cuda.current_device()
+    return torch._C._cuda_getCurrentRawStream(index)

@@ -146,11 +146,12 @@ class ScopePlan:
 
 def _rows2d(x: torch.Tensor, H: int, D: int):
     """(tensor, row stride) of a [rows, H, D] view whose (H, D) part is contiguous"""
-    if x.dim() != 3 or x.shape[1] != H or x.shape[2] != D:
-        raise L.HipValueError(f'expected [rows, {H}, {D}], got {tuple(x.shape)}')
-    if x.stride(2) != 1 or x.stride(1) != D:
+    shape, stride = x.shape, x.stride()   # asked for once: a small layer's time is the host's, this ran nine times in it
+    if len(shape) != 3 or shape[1] != H or shape[2] != D:
+        raise L.HipValueError(f'expected [rows, {H}, {D}], got {tuple(shape)}')
+    if stride[2] != 1 or stride[1] != D:
         raise L.HipValueError('heads and head dims must be contiguous')
-    return x, x.stride(0)
+    return x, stride[0]
 
 
 def _with_row_stride(x: torch.Tensor, stride: int) -> torch.Tensor:
