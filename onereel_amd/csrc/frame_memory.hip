@@ -23,6 +23,7 @@ namespace {
 constexpr int kPoolFly = 32;     // rows per batch of the pooling
 constexpr int kSelThreads = 1024;
 constexpr int kSelWaves = kSelThreads / 64;
+constexpr int kSelRows = 16;      // rows of a column in flight in the member sums
 constexpr int kMaxCand = 1024;
 constexpr int kMaxCentreFloats = 32768;   // k * C: the centres, 128 KiB of LDS
 constexpr int kMaxK = 64;
@@ -76,10 +77,18 @@ __global__ __launch_bounds__(64) void frame_pool_kernel(PoolArgs g) {
   if (col == 0) g.counts[f] += (float)n;
 }
 
-// butterfly sum over the 64 lanes by xor shuffles, the same in every lane
+// sum over the 64 lanes, the same in every lane: the tree of a butterfly with partners 32, 16, 8, 4, 2 and 1 lanes away,
+// on the vector unit (after the first steps the lanes of a row of 16 repeat every 8, 4, .. lanes, so that a rotation
+// reaches the partner's value)
 __device__ __forceinline__ float wave_sum_xor(float v) {
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
+  auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = __uint_as_float(p[0]) + __uint_as_float(p[1]);
+  auto q = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = __uint_as_float(q[0]) + __uint_as_float(q[1]);
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xf, 0xf, false));   // row_ror:8
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x124, 0xf, 0xf, false));   // row_ror:4
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xf, 0xf, false));    // quad_perm 2301
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xf, 0xf, false));    // quad_perm 1032
   return v;
 }
 
@@ -97,11 +106,11 @@ struct SelectArgs {
 };
 
 // two candidate rows against the first `live` (at most NQ) rows of `cv`, C floats apart: acc[i][q] is the lane's share of
-// row i . cv_q, over e = lane, lane + 64, ... in that order. Both rows' loads go out together, 16 steps at a time.
+// row i . cv_q, over e = lane, lane + 64, ... in that order. Both rows' loads go out together, 8 steps at a time.
 template <int NQ>
 __device__ __forceinline__ void dots(const float* x0, const float* x1, const float* cv, int live, int C, int lane,
                                      float (&acc)[2][NQ]) {
-  constexpr int FLY = 16;
+  constexpr int FLY = 8;
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -117,15 +126,17 @@ __device__ __forceinline__ void dots(const float* x0, const float* x1, const flo
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
       if (q >= live) break;
+      float c[FLY];   // no branch around a load: elements past the row multiply zeros
+#pragma unroll
+      for (int u = 0; u < FLY; ++u) c[u] = cv[q * C + min(e0 + 64 * u, C - 1)];
 #pragma unroll
       for (int u = 0; u < FLY; ++u) {
-        const int e = e0 + 64 * u;
-        if (e < C) {
-          const float c = cv[q * C + e];
-          acc[0][q] += a[u] * c;
-          acc[1][q] += b[u] * c;
-        }
+        const bool in = e0 + 64 * u < C;
+        const float cu = in ? c[u] : 0.0f;
+        acc[0][q] += (in ? a[u] : 0.0f) * cu;
+        acc[1][q] += (in ? b[u] : 0.0f) * cu;
       }
+      __builtin_amdgcn_sched_barrier(0);
     }
   }
 }
@@ -153,12 +164,14 @@ __device__ __forceinline__ int wave_argmax(const float* v, int n, int lane) {
 }
 
 // The whole choice in one workgroup: every pass is a few microseconds of dependent loads from the L2, so the passes are
-// few and each keeps many loads in flight: two candidate rows per wavefront and 16 steps of each at once, 16 rows of a
-// column at once in the member sums, and the similarities of the last assignment serve the medoids. Every sum keeps the
-// order of a plain loop over lanes and rows: in a cluster of two, both members are equally similar to their mean, so a
-// sum taken in another order would choose the other one.
+// few and each keeps many loads in flight: two candidate rows per wavefront and 8 steps of each at once, no branch around
+// a load, 16 rows of two columns at once in the member sums (the candidates taken cluster by cluster, so that a row is
+// added once and not to each of eight sums), and the similarities of the last assignment serve the medoids. Every sum
+// keeps the order of a plain loop over lanes and rows: in a cluster of two, both members are equally similar to their
+// mean, so a sum taken in another order would choose the other one.
 // 32 candidates x 2048 columns, 4 centres: 157 us (one 4-byte load at a time per thread, a pass over the candidates and
-// a block-wide argmax tree per medoid) -> 81 us.
+// a block-wide argmax tree per medoid), 81 with the loads batched under branches, sums by selection and shuffles through
+// LDS, now 63 (16 steps at once spilled: 71).
 __global__ __launch_bounds__(kSelThreads) void frame_select_kernel(SelectArgs g, CandTable table) {
   extern __shared__ __attribute__((aligned(16))) float smem[];
   float* c = smem;                  // [k, C] centres
@@ -166,6 +179,7 @@ __global__ __launch_bounds__(kSelThreads) void frame_select_kernel(SelectArgs g,
   __shared__ float dv[kMaxCand];    // per-candidate scores
   __shared__ int z[kMaxCand];       // assignment
   __shared__ int cand[kMaxCand];
+  __shared__ int order[kMaxCand];   // the candidates, cluster by cluster
   __shared__ float sv[8 * kSelWaves];
   __shared__ int centre[kMaxK];
   __shared__ int cnt[kMaxK];
@@ -209,7 +223,7 @@ __global__ __launch_bounds__(kSelThreads) void frame_select_kernel(SelectArgs g,
   // k-means: z = the most similar centre (first on ties); centre i = normalize(mean of its members), unchanged when
   // it has none; stop when no centre changed. After the loop z belongs to the final centres. Centres are taken eight
   // at a time, so that a candidate row is read once per eight dot products and the member sums of eight clusters
-  // accumulate in one pass over the rows (in row order). dv: each candidate's similarity to its centre.
+  // (in row order) are one pass over their rows. dv: each candidate's similarity to its centre.
   for (int it = 0;; ++it) {
     for (int n = 2 * w; n < nc; n += 2 * kSelWaves) {
       float best[2] = {0.0f, 0.0f};
@@ -244,29 +258,52 @@ __global__ __launch_bounds__(kSelThreads) void frame_select_kernel(SelectArgs g,
     if (it == g.iters) break;
     for (int n = tid; n < nc; n += kSelThreads) atomicAdd(&cnt[z[n]], 1);
     __syncthreads();
-    for (int i0 = 0; i0 < k; i0 += 8) {
-      float part[8] = {};
-      for (int e = tid; e < C; e += kSelThreads) {
-        float sum[8] = {};
-        for (int n0 = 0; n0 < nc; n0 += 16) {
-          float v[16];
+    // the candidates cluster by cluster, ascending within one
+    for (int n = tid; n < nc; n += kSelThreads) {
+      int place = 0;
+      for (int i = 0; i < z[n]; ++i) place += cnt[i];
+      for (int m = 0; m < n; ++m) place += z[m] == z[n];
+      order[place] = n;
+    }
+    __syncthreads();
+    for (int i0 = 0, p0 = 0; i0 < k; i0 += 8) {
+      int p1 = p0;     // positions p0 .. p1 - 1 belong to these eight clusters
+      for (int q = 0; q < 8 && i0 + q < k; ++q) p1 += cnt[i0 + q];
+      // the means of their columns, two columns per thread and 16 rows of both at a time, whatever their clusters: a sum
+      // ends where the next position starts another cluster
+      for (int e = tid; e < C; e += 2 * kSelThreads) {
+        const int e1 = min(e + kSelThreads, C - 1);   // past the row: not stored
+        float s0 = 0.0f, s1 = 0.0f;
+        for (int p = p0; p < p1; p += kSelRows) {
+          float v0[kSelRows], v1[kSelRows];
 #pragma unroll
-          for (int u = 0; u < 16; ++u) v[u] = row(n0 + u)[e];
+          for (int u = 0; u < kSelRows; ++u) {
+            const float* x = row(order[min(p + u, p1 - 1)]);
+            v0[u] = x[e];
+            v1[u] = x[e1];
+          }
 #pragma unroll
-          for (int u = 0; u < 16; ++u) {
-            const int zi = n0 + u < nc ? z[n0 + u] - i0 : -1;   // the same for every thread
-#pragma unroll
-            for (int q = 0; q < 8; ++q) sum[q] += zi == q ? v[u] : 0.0f;
+          for (int u = 0; u < kSelRows; ++u) {
+            if (p + u >= p1) break;
+            s0 += v0[u];
+            s1 += v1[u];
+            const int zi = __builtin_amdgcn_readfirstlane(z[order[p + u]]);
+            if (p + u + 1 == p1 || __builtin_amdgcn_readfirstlane(z[order[p + u + 1]]) != zi) {
+              const float n = (float)cnt[zi];
+              mrow[(zi - i0) * C + e] = s0 / n;
+              if (e + kSelThreads < C) mrow[(zi - i0) * C + e1] = s1 / n;
+              s0 = s1 = 0.0f;
+            }
           }
         }
+      }
+      float part[8] = {};
+      for (int e = tid; e < C; e += kSelThreads)
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
-          if (i0 + q >= k) break;
-          const float mean = cnt[i0 + q] ? sum[q] / (float)cnt[i0 + q] : 0.0f;
-          mrow[q * C + e] = mean;
+          const float mean = i0 + q < k && cnt[i0 + q] ? mrow[q * C + e] : 0.0f;   // this thread's own values
           part[q] += mean * mean;
         }
-      }
 #pragma unroll
       for (int q = 0; q < 8; ++q) {
         if (i0 + q >= k) break;
@@ -288,6 +325,7 @@ __global__ __launch_bounds__(kSelThreads) void frame_select_kernel(SelectArgs g,
         }
       }
       __syncthreads();
+      p0 = p1;
     }
     if (!changed) break;   // z and dv were computed from these (unchanged) centres
     __syncthreads();
