@@ -7,7 +7,7 @@
 // centre (the first on ties). Here:
 //
 // - frame_pool_kernel: rows are frame-major (frame of row r = (row0 + r) / T, as the one-GPU processors build
-//   them), so a frame's rows are contiguous. One wavefront per (frame, 128 columns) adds them in row order:
+//   them), so a frame's rows are contiguous. A block per (frame, 128 columns) adds them in row order:
 //   deterministic, unlike an atomic index_add_. Per lane, 2 consecutive columns in fp32.
 // - frame_select_kernel: the whole selection in one workgroup of 1024 threads, centres in LDS (k * C floats); no
 //   host round trip per iteration. Ties are broken towards the lower index, as torch.argmax does. A pass stops when
@@ -20,7 +20,8 @@ namespace onereel {
 
 namespace {
 
-constexpr int kPoolFly = 32;     // rows per batch of the pooling
+constexpr int kPoolThreads = 256;
+constexpr int kPoolRows = 64;    // rows per stage of the pooling
 constexpr int kSelThreads = 1024;
 constexpr int kSelWaves = kSelThreads / 64;
 constexpr int kSelRows = 16;      // rows of a column in flight in the member sums
@@ -36,45 +37,61 @@ struct PoolArgs {
   float* counts;     // [n_frames]
 };
 
-// One wavefront per (frame, 128 columns): a lane owns two columns and adds the frame's rows in row order, so the sums
-// have the same bits whatever the launch. The chain of dependent additions is short (1590 rows: 3 us); what counts are
-// the bytes in flight, so a batch of kPoolFly rows is loaded while the batch before it is added.
-// HBM-bound: eight columns per lane with four rows in flight had 128 wavefronts on the chip and took 168 us for 32
-// frames x 1590 rows x 2048 columns (1.2 TB/s), now 65 us (3.2 TB/s; batches of 64: 69).
-__global__ __launch_bounds__(64) void frame_pool_kernel(PoolArgs g) {
-  const int f = blockIdx.y, col = blockIdx.x * 128 + 2 * threadIdx.x;
+// A block per (frame, 128 columns): its wavefronts load the frame's rows in whole 256-byte pieces, kPoolRows at a time and
+// the next ones in flight, through LDS, and the lanes of the first wavefront, two columns each, add them in row order:
+// the sums have the same bits whatever the launch, and the chain of dependent additions is short (1590 rows: 3 us).
+// HBM-bound, so what counts is the bytes in flight: 32 frames x 1590 rows x 2048 columns took 168 us with eight columns
+// per lane and four rows in flight (128 wavefronts, 1.2 TB/s), 65 with a wavefront per 128 columns that loaded what it
+// added in batches of 32 (of 64: 69), now 33 (6.3 TB/s).
+__global__ __launch_bounds__(kPoolThreads) void frame_pool_kernel(PoolArgs g) {
+  constexpr int PER = kPoolRows * 16 / kPoolThreads;   // 16-byte chunks per thread and stage (16 per row)
+  __shared__ __attribute__((aligned(16))) u32x4 buf[2][kPoolRows][16];
+  const int f = blockIdx.y, col0 = blockIdx.x * 128, tid = threadIdx.x;
   int64_t r0 = (int64_t)f * g.T - g.row0, r1 = r0 + g.T;
   r0 = r0 < 0 ? 0 : r0;
   r1 = r1 > g.n_rows ? g.n_rows : r1;
-  if (r1 <= r0 || col >= g.C) return;
-  const uint16_t* p = g.hs + r0 * g.row_stride + col;
+  if (r1 <= r0) return;
   const int n = (int)(r1 - r0);
+  // this thread's chunk of a row (a chunk past the last column repeats the row's last one; its sums are not stored)
+  const uint16_t* p = g.hs + r0 * g.row_stride + min(col0 + 8 * (tid & 15), g.C - 8);
+  u32x4 v[PER];
+  auto load = [&](int s) {   // stage s, rows past the last repeat it
+#pragma unroll
+    for (int u = 0; u < PER; ++u)
+      v[u] = *(const u32x4*)(p + (int64_t)min(s * kPoolRows + u * (kPoolThreads / 16) + (tid >> 4), n - 1) * g.row_stride);
+  };
   float a0 = 0.0f, a1 = 0.0f;
-  uint32_t v[2][kPoolFly];
-  auto load = [&](int b, uint32_t (&x)[kPoolFly]) {   // batch b, rows past the last repeat it
+  const int stages = (n + kPoolRows - 1) / kPoolRows;
+  load(0);
+  for (int s = 0; s < stages; ++s) {
 #pragma unroll
-    for (int u = 0; u < kPoolFly; ++u) x[u] = *(const uint32_t*)(p + (int64_t)min(b * kPoolFly + u, n - 1) * g.row_stride);
-  };
-  auto add = [&](int b, const uint32_t (&x)[kPoolFly]) {
+    for (int u = 0; u < PER; ++u) buf[s & 1][u * (kPoolThreads / 16) + (tid >> 4)][tid & 15] = v[u];
+    if (s + 1 < stages) load(s + 1);
+    __syncthreads();   // stage s is there; the sums of stage s - 2 in this half are long done (the barrier before)
+    if (tid < 64) {
+      const uint32_t* x = (const uint32_t*)&buf[s & 1][0][0] + tid;
+      const int rows = min(kPoolRows, n - s * kPoolRows);
+      if (rows == kPoolRows) {
 #pragma unroll
-    for (int u = 0; u < kPoolFly; ++u)
-      if (b * kPoolFly + u < n) {
-        a0 += bf2f((uint16_t)(x[u] & 0xffffu));
-        a1 += bf2f((uint16_t)(x[u] >> 16));
+        for (int r = 0; r < kPoolRows; ++r) {
+          a0 += bf2f((uint16_t)(x[64 * r] & 0xffffu));
+          a1 += bf2f((uint16_t)(x[64 * r] >> 16));
+        }
+      } else {
+        for (int r = 0; r < rows; ++r) {
+          a0 += bf2f((uint16_t)(x[64 * r] & 0xffffu));
+          a1 += bf2f((uint16_t)(x[64 * r] >> 16));
+        }
       }
-  };
-  const int batches = (n + kPoolFly - 1) / kPoolFly;
-  load(0, v[0]);
-  for (int b = 0; b < batches; b += 2) {
-    load(min(b + 1, batches - 1), v[1]);
-    add(b, v[0]);
-    load(min(b + 2, batches - 1), v[0]);
-    add(b + 1, v[1]);
+    }
   }
-  float* sp = g.sums + (int64_t)f * g.C + col;
-  sp[0] += a0;
-  sp[1] += a1;
-  if (col == 0) g.counts[f] += (float)n;
+  const int col = col0 + 2 * tid;
+  if (tid < 64 && col < g.C) {
+    float* sp = g.sums + (int64_t)f * g.C + col;
+    sp[0] += a0;
+    sp[1] += a1;
+    if (col == 0) g.counts[f] += (float)n;
+  }
 }
 
 // sum over the 64 lanes, the same in every lane: the tree of a butterfly with partners 32, 16, 8, 4, 2 and 1 lanes away,
@@ -382,7 +399,7 @@ extern "C" int or_frame_pool(const void* hs, int64_t n_rows, int32_t C, int64_t 
                     n_frames);
   if (((uintptr_t)hs & 15u) || row_stride % 8) return fail_arg("or_frame_pool: hs must be 16-byte aligned rows");
   PoolArgs g{(const uint16_t*)hs, n_rows, row_stride, row0, C, T, n_frames, sums, counts};
-  hipLaunchKernelGGL(frame_pool_kernel, dim3((unsigned)((C + 127) / 128), (unsigned)n_frames), dim3(64), 0,
+  hipLaunchKernelGGL(frame_pool_kernel, dim3((unsigned)((C + 127) / 128), (unsigned)n_frames), dim3(kPoolThreads), 0,
                      (hipStream_t)stream, g);
   return check_hip(hipGetLastError(), "frame_pool_kernel launch");
 }
