@@ -200,9 +200,8 @@ def ptr(t):
 def device_ints(lists, device):
     """lists of Python ints as int32 tensors on the device: parts of one tensor, filled by launches that carry the
     values (a copy from pageable memory would cost each list about 10 us of the host's time)"""
-    device = torch.device(device)
     flat = [int(x) for values in lists for x in values]
-    if device.type != 'cuda' or not flat or min(flat) < -2 ** 31 or max(flat) >= 2 ** 31:
+    if device is None or torch.device(device).type != 'cuda' or not flat or min(flat) < -2 ** 31 or max(flat) >= 2 ** 31:
         return [torch.tensor(list(values), dtype=torch.int32, device=device) for values in lists]
     out = torch.empty(len(flat), dtype=torch.int32, device=device)
     with torch.cuda.device(out.device):
@@ -214,7 +213,7 @@ def device_ints(lists, device):
 def stream_handle(device=None):
     """the current stream of the device (default: the current one), as a handle. The Stream object that
     torch.cuda.current_stream makes for it costs more than a launch's arguments."""
-    index = device.index if isinstance(device, torch.device) else device
+    index = device if device is None or isinstance(device, int) else torch.device(device).index
     if index is None:
         index = torch.cuda.current_device()
     return torch._C._cuda_getCurrentRawStream(index)
