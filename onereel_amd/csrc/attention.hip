@@ -1285,22 +1285,24 @@ __global__ __launch_bounds__(kThreads) void merge_kernel(AttnArgs a, const int32
 // HBM, and the item machinery of attn8_kernel (a ring fill, an epilogue and a claim per 256 queries, for 4 key blocks
 // of matrix work) is what it spends its time on. Here a block loads a segment-head's K and V into LDS once (LDS DMA,
 // swizzled as in the ring kernels) and its wavefronts stream the queries past them, 32 at a time and independently of
-// each other: no barrier after the load, the next 32 queries in flight while this tile computes, the scores of 128 keys
-// in registers at once (one max, no running rescale up to 128 keys), the output through LDS so that a row's 128-byte
-// lines are stored whole. Two wavefronts per SIMD: NB = 4 (128 keys, 80 KB of LDS) two blocks of 4 wavefronts per CU,
-// NB = 8 (256 keys, 160 KB) one block of 8.
+// each other: no barrier after the load, the next 32 queries in flight while this tile computes, the output through LDS
+// so that a row's 128-byte lines are stored whole. Two wavefronts per SIMD: NB = 4 (128 keys, 80 KB of LDS) two blocks
+// of 4 wavefronts per CU, NB = 8 (256 keys, 160 KB) one block of 8.
 // A block finds its item (query range of a segment, head) from cu_q by itself, so there is no planner launch; items of
 // the same rows and consecutive heads run side by side, so that whole q / o rows stream through.
-// Measured against the ring kernel with its planner (with lse): 16 x 13 200 queries x 24 heads, 64 keys 1000 -> 550 us
-// (4.7 TB/s; a device copy reaches 5.5), 128 keys 1090 -> 570, 200 keys 1240 -> 795, 256 keys 1285 -> 865; 880 + 1100 +
-// 880 queries x 24 heads, 128 keys 54 (planner, attention and merge kernels) -> 14. Between 128 and 256 keys the matrix and vector work of a
-// CU (one block of 8 wavefronts) is as long as the stream. 256 to 2048 queries per item measured alike.
-// Past 128 keys the scores of a tile don't fit the registers beside O: chunks of up to 3 blocks, whose running max moves
-// only when a probability would pass 2^kShortRaise (chunks of 4 spilled: 1450 us at 256 keys).
+// The arithmetic is attn8_kernel's, operation for operation: the running max starts at the first block's, later scores
+// accumulate onto -m, a block's row sum is added in the same order, O is scaled by the hardware reciprocal. So a segment's
+// O and lse have the same bits whichever kernel the call's max_k selects (unless the planner splits items by keys there,
+// or a sum of probabilities passes 2^20: the max then moves for the 32 queries of a tile here, for 64 there). An exact
+// maximum over up to 128 keys at once rounds P elsewhere: other bits, and no faster.
+// Measured against the ring kernel with its planner (with lse): 16 x 13 200 queries x 24 heads, 64 keys 1000 -> 540 us
+// (4.8 TB/s; a device copy reaches 5.5), 128 keys 1090 -> 555, 200 keys 1240 -> 725, 256 keys 1285 -> 795; 880 + 1100 +
+// 880 queries x 24 heads, 128 keys 54 (planner, attention and merge kernels) -> 13. Between 128 and 256 keys the matrix
+// and vector work of a CU (one block of 8 wavefronts) is as long as the stream. 256 to 2048 queries per item measured
+// alike. Past 256 keys K and V of a head no longer fit the LDS.
 constexpr int kShortKeys = 256;
 constexpr int kShortSegs = 256;   // a block finds its segment 64 at a time
-
-constexpr float kShortRaise = 16.0f;   // log2 of the largest probability kept relative to an older max
+constexpr int kShortSlot = kBKB * 128 * 2;   // bytes of a K or V block in LDS
 
 // LDS byte addresses of this lane's operands in slot 0: K step k (8), V^T rows of 32 dims db (4). Every read is one of
 // them plus a constant that fits the instruction's offset (formed from one base per read they took 60 registers).
@@ -1311,71 +1313,94 @@ struct ShortLds {
 struct ShortTile {
   bf16x8 q[8];
   f32x16 acc[4];
+  f32x16 neg;   // -m, 16 times: the scores of every block past the first accumulate onto it
   float m, l;
 };
 
-// one chunk of N key blocks (the segment's last block among them when `valid` < 16: this lane half's keys there) of a
-// 32-query tile: scores, softmax against the chunks before (FIRST: none), PV. qnext: this lane's next query, loaded
-// into t.q once the scores are done with it (nullptr: not the tile's last chunk).
-template <int N, bool FIRST>
-__device__ __forceinline__ void short_chunk(ShortTile& t, const ShortLds& ad, const int b0, int valid, float c,
-                                            const uint16_t* qnext) {
-  constexpr int SLOT = kBKB * 128 * 2;   // bytes
-  typedef __attribute__((address_space(3))) char lds_char;
+typedef __attribute__((address_space(3))) char lds_char;
+
+// key block `slot`'s scores, accumulated onto `seed`; keys from `valid` on (this lane half's keys of the block) masked
+__device__ __forceinline__ f32x16 short_scores(const ShortTile& t, const ShortLds& ad, int slot, int valid,
+                                               const f32x16& seed) {
   typedef __attribute__((address_space(3))) const bf16x8 lds_bf16x8;
-  typedef __attribute__((address_space(3))) bf16x4 lds_bf16x4;
-  f32x16 s[N];
+  f32x16 s = seed;
 #pragma unroll
-  for (int b = 0; b < N; ++b) {
-    const f32x16 zero = {};
-#pragma unroll
-    for (int k = 0; k < 8; ++k)
-      s[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(lds_bf16x8*)((lds_char*)(uintptr_t)ad.k[k] + (b0 + b) * SLOT),
-                                                     t.q[k], k == 0 ? zero : s[b], 0, 0, 0);
-    if (!FIRST || N == 4) __builtin_amdgcn_sched_barrier(0);
-  }
-  if (qnext)
-#pragma unroll
-    for (int k = 0; k < 8; ++k) t.q[k] = as_bf16x8(*(const u32x4*)(qnext + 16 * k));
+  for (int k = 0; k < 8; ++k)
+    s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(lds_bf16x8*)((lds_char*)(uintptr_t)ad.k[k] + slot * kShortSlot),
+                                                t.q[k], s, 0, 0, 0);
   if (valid < 16)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) s[N - 1][r] = r < valid ? s[N - 1][r] : -__builtin_inff();
-  float mx = max16(s[0]);
+    for (int r = 0; r < 16; ++r) s[r] = r < valid ? s[r] : -__builtin_inff();
+  return s;
+}
+
+// the first block's scores set the running max; they become relative to it
+__device__ __forceinline__ void short_start(ShortTile& t, f32x16& s) {
+  t.m = pair_max(max16(s));
+  t.l = 0.0f;
 #pragma unroll
-  for (int b = 1; b < N; ++b) mx = fmaxf(mx, max16(s[b]));
-  mx = pair_max(mx);
-  if constexpr (FIRST) {
-    t.m = mx;
-    t.l = 0.0f;
-  } else if (__any(!((mx - t.m) * c <= kShortRaise))) {
-    // the running max moves only when some probability would exceed 2^kShortRaise (O and l stay relative to it)
-    const float mn = fmaxf(t.m, mx);
-    const float alpha = __builtin_amdgcn_exp2f((t.m - mn) * c);
+  for (int r = 0; r < 16; ++r) {
+    s[r] -= t.m;
+    t.neg[r] = -t.m;
+  }
+}
+
+// P = 2^(c s) rounded to bf16 pairs and the fp32 sum of the unrounded values, in the order in which the ring kernel's
+// key loop adds them
+__device__ __forceinline__ float short_probs(const f32x16& s, float c, bf16x8 (&p)[2]) {
+  float e[16], t[8];
+#pragma unroll
+  for (int r = 0; r < 16; ++r) e[r] = __builtin_amdgcn_exp2f(c * s[r]);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) t[i] = e[2 * i] + e[2 * i + 1];
+#pragma unroll
+  for (int half = 0; half < 2; ++half) {
+    u32x4 pk;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) pk[i] = pack2(e[8 * half + 2 * i], e[8 * half + 2 * i + 1]);
+    p[half] = as_bf16x8(pk);
+  }
+  return ((t[0] + t[4]) + (t[1] + t[5])) + ((t[2] + t[6]) + (t[3] + t[7]));
+}
+
+// softmax and PV of one key block whose scores (relative to the running max) are s; `next`: the scores of the block after
+// it, already computed (or this block's own where there is none). FIRST: no block before it.
+template <bool FIRST>
+__device__ __forceinline__ void short_block(ShortTile& t, const ShortLds& ad, int slot, f32x16& s, f32x16& next,
+                                            float c) {
+  typedef __attribute__((address_space(3))) bf16x4 lds_bf16x4;
+  bf16x8 p[2];
+  float ls = short_probs(s, c, p);
+  if (!FIRST && __any(!(ls <= kRescaleSum))) {
+    // the running max moves up by d: O and l scale by 2^(-c d), the scores taken relative to the old one shift
+    const float d = fmaxf(pair_max(max16(s)), 0.0f);
+    const float alpha = __builtin_amdgcn_exp2f(-(c * d));
+    t.m += d;
+    t.l *= alpha;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      s[r] -= d;
+      next[r] -= d;
+      t.neg[r] -= d;
+    }
 #pragma unroll
     for (int db = 0; db < 4; ++db)
 #pragma unroll
       for (int r = 0; r < 16; ++r) t.acc[db][r] *= alpha;
-    t.l *= alpha;
-    t.m = mn;
+    ls = short_probs(s, c, p);
   }
-  const float mc = t.m * c;
+  t.l += ls;
 #pragma unroll
-  for (int b = 0; b < N; ++b) {
-    bf16x8 p[2];
-    t.l += exp_pack(s[b], c, mc, p);
-    __builtin_amdgcn_sched_barrier(0);
+  for (int half = 0; half < 2; ++half)
 #pragma unroll
-    for (int half = 0; half < 2; ++half)
-#pragma unroll
-      for (int db = 0; db < 4; ++db) {
-        const f32x16 zero = {};
-        lds_char* at = (lds_char*)(uintptr_t)ad.v[db] + (b0 + b) * SLOT + 8 * half * 256;
-        const u32x2 lo = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)at));
-        const u32x2 hi = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)(at + 4 * 256)));
-        t.acc[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(u32x4{lo[0], lo[1], hi[0], hi[1]}), p[half],
-                                                            FIRST && b == 0 && half == 0 ? zero : t.acc[db], 0, 0, 0);
-      }
-  }
+    for (int db = 0; db < 4; ++db) {
+      const f32x16 zero = {};
+      lds_char* at = (lds_char*)(uintptr_t)ad.v[db] + slot * kShortSlot + 8 * half * 256;
+      const u32x2 lo = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)at));
+      const u32x2 hi = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)(at + 4 * 256)));
+      t.acc[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(u32x4{lo[0], lo[1], hi[0], hi[1]}), p[half],
+                                                          FIRST && half == 0 ? zero : t.acc[db], 0, 0, 0);
+    }
 }
 
 // a block's item: `rows` queries from packed query q0 on, of a segment with Lk keys
@@ -1393,7 +1418,7 @@ __device__ __forceinline__ const uint16_t* short_q(const AttnArgs& a, const Shor
 __device__ __forceinline__ void short_store(const AttnArgs& a, const ShortItem& x, const ShortTile& t, int tt, int lane,
                                             uint16_t* st) {
   const int l32 = lane & 31, h = lane >> 5;
-  const float ltot = pair_sum(t.l), inv = x.Lk > 0 ? 1.0f / ltot : 0.0f;
+  const float ltot = pair_sum(t.l), inv = x.Lk > 0 ? __builtin_amdgcn_rcpf(ltot) : 0.0f;
   if (a.lse && h == 0 && 32 * tt + l32 < x.rows)
     a.lse[(int64_t)x.head * a.sum_q + x.q0 + 32 * tt + l32] =
         x.Lk > 0 ? t.m * a.scale + logf(ltot) : -__builtin_inff();
@@ -1424,27 +1449,39 @@ __device__ __forceinline__ void short_store(const AttnArgs& a, const ShortItem& 
 template <int NBC, int NW>
 __device__ __forceinline__ void short_tiles(const AttnArgs& a, const ShortItem& x, const ShortLds& ad, int w, int lane,
                                             uint16_t* st) {
-  // up to 4 blocks in one chunk; more in chunks of up to 3 (their scores beside the live accumulators)
-  constexpr int N0 = NBC <= 4 ? NBC : 3, N1 = NBC <= 4 ? 0 : NBC <= 6 ? NBC - 3 : NBC - 5, N2 = NBC - N0 - N1;
   const int l32 = lane & 31, h = lane >> 5;
   const int valid = x.Lk - (NBC - 1) * kBKB - 16 * h;
+  const f32x16 zero = {};
   ShortTile t;
   const uint16_t* qp = short_q(a, x, w, l32, h);
 #pragma unroll
   for (int k = 0; k < 8; ++k) t.q[k] = as_bf16x8(*(const u32x4*)(qp + 16 * k));
   for (int tt = w; 32 * tt < x.rows; tt += NW) {
     const uint16_t* qn = short_q(a, x, tt + NW, l32, h);
-    if constexpr (N1 == 0) {
-      short_chunk<N0, true>(t, ad, 0, valid, a.c, qn);
-    } else {
-      short_chunk<N0, true>(t, ad, 0, 16, a.c, nullptr);
-      if constexpr (N2 == 0) {
-        short_chunk<N1, false>(t, ad, N0, valid, a.c, qn);
-      } else {
-        short_chunk<N1, false>(t, ad, N0, 16, a.c, nullptr);
-        short_chunk<N2, false>(t, ad, N0 + N1, valid, a.c, qn);
-      }
+    // the next tile's queries: in flight during the whole tile where the registers allow it (two to four blocks, 64 to
+    // 128 keys of 16 x 13 200 queries x 24 heads: 545 to 569 us with the loads behind the last scores, 538 to 553 so)
+    constexpr bool kEarly = NBC > 1 && NBC <= 4;
+    bf16x8 qnext[8];
+    auto load_next = [&] {
+#pragma unroll
+      for (int k = 0; k < 8; ++k) qnext[k] = as_bf16x8(*(const u32x4*)(qn + 16 * k));
+    };
+    if constexpr (kEarly) {
+      load_next();
+      __builtin_amdgcn_sched_barrier(0);
     }
+    f32x16 s[2];   // block b in s[b % 2]: the next block's scores are computed ahead of a block's softmax
+    s[0] = short_scores(t, ad, 0, NBC == 1 ? valid : 16, zero);
+    short_start(t, s[0]);
+#pragma unroll
+    for (int b = 0; b < NBC; ++b) {
+      if (b + 1 < NBC) s[(b + 1) & 1] = short_scores(t, ad, b + 1, b + 2 == NBC ? valid : 16, t.neg);
+      if (!kEarly && (b + 2 == NBC || NBC == 1)) load_next();   // behind the tile's last scores
+      if (b == 0) short_block<true>(t, ad, b, s[0], s[1], a.c);
+      else short_block<false>(t, ad, b, s[b & 1], s[(b + 1) & 1], a.c);
+    }
+#pragma unroll
+    for (int k = 0; k < 8; ++k) t.q[k] = qnext[k];
     short_store(a, x, t, tt, lane, st);
   }
 }
@@ -1530,7 +1567,7 @@ void attn_short_kernel(AttnArgs a, int n_seg, int item_rows) {
     const uint16_t* qp = short_q(a, x, t0 + w, l32, h);
 #pragma unroll
     for (int k = 0; k < 8; ++k) t.q[k] = as_bf16x8(*(const u32x4*)(qp + 16 * k));
-    t.m = kMInit;
+    t.m = 0.0f;
     t.l = 0.0f;
 #pragma unroll
     for (int db = 0; db < 4; ++db)
@@ -1540,7 +1577,10 @@ void attn_short_kernel(AttnArgs a, int n_seg, int item_rows) {
       __syncthreads();
       load_blocks(b, 1);
       wait_loads_barrier<0>();
-      short_chunk<1, false>(t, ad, 0, x.Lk - b * kBKB - 16 * h, a.c, nullptr);
+      const f32x16 zero = {};
+      f32x16 s = short_scores(t, ad, 0, x.Lk - b * kBKB - 16 * h, b == 0 ? zero : t.neg), none = zero;
+      if (b == 0) short_start(t, s);
+      short_block<false>(t, ad, 0, s, none, a.c);
     }
     short_store(a, x, t, t0 + w, lane, st);
   }
@@ -1664,10 +1704,9 @@ int check_args(const or_varlen_args& x, const char* fn) {
 }
 
 // calls that attn_short_kernel runs: at most 256 keys per segment (K and V of a head in 128 KB of LDS), without the
-// options that only the ring kernels have (queries named by source row among them: a scene layer's calls, which give the
-// same bits with their values packed or read in place, stay on one kernel), and with few enough segments that finding one is cheap (256 segments of 10
-// queries x 24 heads: 172 -> 62 us; each further 64 cost every block another look at cu_q). Segments longer than max_k
-// says still come out right (streamed block by block for every tile).
+// options that only the ring kernels have (queries named by source row among them), and with few enough segments that
+// finding one is cheap (256 segments of 10 queries x 24 heads: 172 -> 62 us; each further 64 cost every block another look
+// at cu_q). Segments longer than max_k says still come out right (streamed block by block for every tile).
 bool short_keys(const or_varlen_args& x) {
   return x.D == 128 && x.max_k >= 1 && x.max_k <= kShortKeys && x.n_seg <= kShortSegs && !x.seg_q_src && !x.q_rope &&
          !x.k_len_head && !x.v_tok && !x.k_tok;
