@@ -370,7 +370,7 @@ int or_memory_foreign(const int64_t* rep, const uint8_t* valid, const int64_t* c
                       int32_t* k_len_head, void* stream);
 
 /* n int32 values of host memory into device memory by kernel launches that carry them (896 each): no copy, and the host
- * array is free on return. */
+ * array is free on return. The values are there for later work of `stream`; another stream has to wait for it. */
 int or_index_fill(const int32_t* values, int32_t n, int32_t* out, void* stream);
 
 /* The concatenations and offsets of attention.packed (src/onereel/attention.py:56-71): n_seg sequences of nq[s] query and

@@ -199,7 +199,9 @@ def ptr(t):
 
 def device_ints(lists, device):
     """lists of Python ints as int32 tensors on the device: parts of one tensor, filled by launches that carry the
-    values (a copy from pageable memory would cost each list about 10 us of the host's time)"""
+    values (a copy from pageable memory would cost each list about 10 us of the host's time). The launches are queued on
+    the device's current stream and not waited for: for a call that reads the values on that stream, not for tensors
+    that are handed out"""
     flat = [int(x) for values in lists for x in values]
     if device is None or torch.device(device).type != 'cuda' or not flat or min(flat) < -2 ** 31 or max(flat) >= 2 ** 31:
         return [torch.tensor(list(values), dtype=torch.int32, device=device) for values in lists]

@@ -33,3 +33,19 @@ def test_concat(n, H, D, most):
     # rows that are not contiguous are concatenated by torch: the same tensors
     wide = [(torch.cat([q, q], 2)[..., :D], k, v) for q, k, v in seg]
     assert torch.equal(A._concat(wide)[0][0], q) and torch.equal(A._concat(wide)[0][3], cu_q)
+
+
+def test_cu_seqlens_are_there_on_return():
+    """offsets handed out are read on other streams without an event between: they are filled when the call returns, also
+    behind work that its own stream has still to do"""
+    want = [3 * i for i in range(513)]
+    junk = torch.full((513,), -1, dtype=torch.int32, device=DEV)   # what the offsets' allocation holds before
+    torch.cuda.synchronize()
+    del junk
+    side = torch.cuda.Stream()
+    torch.cuda._sleep(200_000_000)
+    cu = A.cu_seqlens([3] * 512, DEV)
+    with torch.cuda.stream(side):
+        got = cu.cpu()
+    torch.cuda.synchronize()
+    assert got.tolist() == want
