@@ -214,8 +214,14 @@ def device_ints(lists, device):
 
 def stream_handle(device=None):
     """the current stream of the device (default: the current one), as a handle. The Stream object that
-    torch.cuda.current_stream makes for it costs more than a launch's arguments."""
-    index = device if device is None or isinstance(device, int) else torch.device(device).index
+    torch.cuda.current_stream makes for it costs more than a launch's arguments. A device that is no GPU is refused, as
+    there: the entry points that check nothing else about their tensors' device stop here, ahead of the launch."""
+    index = device
+    if device is not None and not isinstance(device, int):
+        device = torch.device(device)
+        if device.type != 'cuda':
+            raise ValueError(f'Expected a cuda device, but got: {device}')
+        index = device.index
     if index is None:
         index = torch.cuda.current_device()
     return torch._C._cuda_getCurrentRawStream(index)

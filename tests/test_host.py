@@ -515,3 +515,33 @@ def test_drop_in_varlen_rejects_bad_offsets_and_ranges_without_gpu():
         A.overlapping_ranges(q, k, k, [(0, 4), (4, 10)], [(5, 3), (0, 2)])
     with pytest.raises(L.HipValueError, match='pair up'):
         A.overlapping_ranges(q, k, k, [(0, 4), (4, 10)], [(0, 6)])
+
+
+def test_tensors_off_the_gpu_are_refused_ahead_of_the_launch(monkeypatch):
+    """the entry points that look at no device themselves hand their tensors' device to stream_handle: a CPU tensor's must
+    not give the GPU's current stream"""
+    from onereel_amd import attention as A
+    from onereel_amd import wan as W
+    from onereel_amd import wan_dit as WD
+    monkeypatch.setattr(torch.cuda, 'current_device', lambda: 0)
+    monkeypatch.setattr(torch._C, '_cuda_getCurrentRawStream', lambda index: index, raising=False)
+    for device in ('cpu', torch.device('cpu'), 'meta'):
+        with pytest.raises(ValueError, match='cuda device'):
+            L.stream_handle(device)
+    assert [L.stream_handle(d) for d in (None, 3, 'cuda', 'cuda:2', torch.device('cuda:1'))] == [0, 3, 0, 2, 1]
+
+    class NoLaunch:
+        def __getattr__(self, name):
+            return lambda *a: pytest.fail(f'{name} was called with CPU tensors')
+
+    monkeypatch.setattr(L, 'lib', lambda: NoLaunch())
+    monkeypatch.setattr(L, 'dit_lib', lambda: NoLaunch())
+    bf16 = lambda *s: torch.zeros(*s, dtype=torch.bfloat16)
+    calls = [lambda: W.rms_norm(bf16(4, 512), bf16(512), 1e-6),
+             lambda: W._qk(bf16(4, 512), bf16(4, 512), bf16(512), bf16(512), 1e-6, torch.zeros(4, 128),
+                           torch.zeros(4, 128), 4),
+             lambda: A.merge_lse(torch.zeros(4, 2, 128), torch.zeros(2, 4), bf16(4, 2, 128), torch.zeros(2, 4)),
+             lambda: WD.layernorm_modulate(bf16(4, 512), 1e-6)]
+    for call in calls:
+        with pytest.raises(ValueError, match='cuda device'):
+            call()
