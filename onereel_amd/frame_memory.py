@@ -10,6 +10,8 @@ of a fallback layout. One GPU holds every token, so the per-frame sums need no a
 """
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import torch
 import torch.nn.functional as F
@@ -187,10 +189,12 @@ class FrameMemory:
         reps = torch.empty(k, dtype=torch.int32, device=dev)
         work = torch.empty(8, C, dtype=torch.float32, device=dev)
         if n_frames <= 65536:
-            # the candidates travel with the launch
-            fn, ct = L.lib().or_frame_select_host, torch.tensor(cand, dtype=torch.int32)
+            # the candidates travel with the launch, from host memory (a ctypes array: a tensor without a device goes to
+            # torch's default device)
+            fn, ct = L.lib().or_frame_select_host, (ctypes.c_int32 * len(cand))(*cand)
         else:
-            fn, ct = L.lib().or_frame_select, torch.tensor(cand, dtype=torch.int32, device=dev)
-        L.check(fn(x.data_ptr(), n_frames, C, ct.data_ptr(), len(cand), k, self.iters, reps.data_ptr(),
+            on_gpu = torch.tensor(cand, dtype=torch.int32, device=dev)
+            fn, ct = L.lib().or_frame_select, on_gpu.data_ptr()
+        L.check(fn(x.data_ptr(), n_frames, C, ct, len(cand), k, self.iters, reps.data_ptr(),
                    work.data_ptr(), L.stream_handle(dev)), 'or_frame_select')
         return [int(r) for r in reps.cpu().tolist() if r >= 0]

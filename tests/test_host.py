@@ -545,3 +545,21 @@ def test_tensors_off_the_gpu_are_refused_ahead_of_the_launch(monkeypatch):
     for call in calls:
         with pytest.raises(ValueError, match='cuda device'):
             call()
+
+
+@pytest.mark.parametrize('default', ['cpu', 'meta'])
+def test_frame_select_hands_over_candidates_in_host_memory(monkeypatch, default):
+    """under any default device of torch's: the library reads the array on the host"""
+    class Lib:
+        @staticmethod
+        def or_frame_select_host(feats, n, C, cand, n_cand, k, iters, reps, work, stream):
+            ctypes.memmove(reps, cand, 4 * k)   # reads the candidates on the host
+            return 0
+
+    monkeypatch.setattr(L, 'lib', lambda: Lib)
+    monkeypatch.setattr(L, 'stream_handle', lambda device=None: 0)
+    fm = FrameMemory(budget=3)
+    fm.reset(SceneLayout([4, 3], halo=0), 2)
+    feats = torch.randn(7, 16, device='cpu')
+    with torch.device(default):
+        assert fm.select(feats) == fm.candidate_frames()[:3] == [0, 1, 2]
