@@ -330,8 +330,12 @@ int or_frame_select(const float* feats, int32_t n_frames, int32_t C, const int32
 int or_frame_select_host(const float* feats, int32_t n_frames, int32_t C, const int32_t* cand, int32_t n_cand,
                          int32_t k, int32_t iters, int32_t* reps, float* work, void* stream);
 
-/* Bytes of device workspace or_memory_select needs: the normalised keys [H, B, D] fp32 and per-candidate arrays. */
+/* Bytes of device workspace or_memory_select needs for keys of either type: per-candidate and per-centroid arrays and,
+ * for fp32 keys, the normalised keys [H, B, D]. */
 int64_t or_memory_select_workspace_size(int32_t B, int32_t H, int32_t D, int32_t M, int32_t iters);
+
+/* The same for keys of one type: bf16 keys (fp32_keys 0) are read where they are and need none of H * B * D * 4 bytes. */
+int64_t or_memory_select_workspace_bytes(int32_t B, int32_t H, int32_t D, int32_t M, int32_t iters, int32_t fp32_keys);
 
 /* Replaces BoundaryMemory.select (src/onereel/memory.py:58-93): per head h, k-means over the B candidate keys
  * x_b = key_b / max(|key_b|, 1e-12) (key_b: row rows[b] (or b) of keys, head h, D elements; bf16, or fp32 when

@@ -85,6 +85,7 @@ SIGNATURES = {
     'or_frame_select_host': (i32, [vp, i32, i32, vp, i32, i32, i32, vp, vp, vp]),
     'or_frame_select': (i32, [vp, i32, i32, vp, i32, i32, i32, vp, vp, vp]),
     'or_memory_select_workspace_size': (i64, [i32, i32, i32, i32, i32]),
+    'or_memory_select_workspace_bytes': (i64, [i32, i32, i32, i32, i32, i32]),
     'or_memory_select': (i32, [vp, i32, vp, i64, i32, i32, i32, i32, vp, vp, i32, vp, vp, vp, i64, vp]),
     'or_memory_index': (i32, [vp, vp, vp, vp, vp, vp, vp, vp, i32, i32, i32, vp, vp, vp]),
     'or_memory_foreign': (i32, [vp, vp, vp, vp, vp, vp, vp, vp, i32, i32, i32, vp, vp, vp, vp]),

@@ -51,7 +51,7 @@ struct SelArgs {
   const int32_t* rows;      // [B] row of each candidate in keys (NULL: candidate b is row b)
   int64_t stride;           // elements between consecutive rows of keys
   int B, H, D, M, fp32_in, iters;
-  float* X;                 // [H, B, D] normalised keys (fp32 keys only)
+  float* X;                 // [H, B, D] normalised keys (fp32 keys only: bf16 keys have no room for it)
   float* inv;               // [H, B] 1 / max(|key|, 1e-12)
   float* xx;                // [H, B] |x|^2
   float* C;                 // [H, M, D] centroids (in / out)
@@ -629,7 +629,8 @@ struct WsParts {
   int64_t X, inv, xx, cc, z, dist, moved, total;
 };
 
-WsParts ws_parts(int B, int H, int D, int M, int iters) {
+// (bf16 keys need no X)
+WsParts ws_parts(int B, int H, int D, int M, int iters, bool fp32_keys) {
   WsParts p;
   int64_t o = 0;
   auto take = [&](int64_t bytes) {
@@ -637,7 +638,7 @@ WsParts ws_parts(int B, int H, int D, int M, int iters) {
     o += (bytes + 255) / 256 * 256;
     return at;
   };
-  p.X = take((int64_t)H * B * D * 4);
+  p.X = take(fp32_keys ? (int64_t)H * B * D * 4 : 0);
   p.inv = take((int64_t)H * B * 4);
   p.xx = take((int64_t)H * B * 4);
   p.cc = take((int64_t)H * M * 4);
@@ -653,9 +654,14 @@ WsParts ws_parts(int B, int H, int D, int M, int iters) {
 
 using namespace onereel;
 
-extern "C" int64_t or_memory_select_workspace_size(int32_t B, int32_t H, int32_t D, int32_t M, int32_t iters) {
+extern "C" int64_t or_memory_select_workspace_bytes(int32_t B, int32_t H, int32_t D, int32_t M, int32_t iters,
+                                                    int32_t fp32_keys) {
   if (B < 1 || H < 1 || M < 1 || iters < 0 || (D != 64 && D != 128)) return -1;
-  return ws_parts(B, H, D, M, iters).total;
+  return ws_parts(B, H, D, M, iters, fp32_keys != 0).total;
+}
+
+extern "C" int64_t or_memory_select_workspace_size(int32_t B, int32_t H, int32_t D, int32_t M, int32_t iters) {
+  return or_memory_select_workspace_bytes(B, H, D, M, iters, 1);
 }
 
 extern "C" int or_memory_select(const void* keys, int32_t fp32_keys, const int32_t* rows, int64_t key_row_stride,
@@ -669,7 +675,7 @@ extern "C" int or_memory_select(const void* keys, int32_t fp32_keys, const int32
   if (iters < 0 || iters > 1000) return fail_arg("or_memory_select: iters=%d outside [0, 1000]", iters);
   if (!keys || !centroids || !rep || !valid || key_row_stride < (int64_t)H * D)
     return fail_arg("or_memory_select: keys, centroids, rep and valid are required, rows of at least H*D elements");
-  const WsParts wp = ws_parts(B, H, D, M, iters);
+  const WsParts wp = ws_parts(B, H, D, M, iters, fp32_keys != 0);
   if (!workspace || workspace_bytes < wp.total || ((uintptr_t)workspace & 255u))
     return fail_arg("or_memory_select: a 256-byte aligned workspace of %lld bytes is needed", (long long)wp.total);
   if (((uintptr_t)centroids & 15u) || ((uintptr_t)keys & 15u) || key_row_stride % (fp32_keys ? 4 : 8))

@@ -79,8 +79,8 @@ class BoundaryMemory:
             self._init_cols[key] = cols.to(device)
         return self._init_cols[key]
 
-    def _workspace(self, B, H, D, M, iters, device):
-        n = int(L.lib().or_memory_select_workspace_size(B, H, D, M, iters))
+    def _workspace(self, B, H, D, M, iters, fp32_keys, device):
+        n = int(L.lib().or_memory_select_workspace_bytes(B, H, D, M, iters, fp32_keys))
         if n < 0:
             raise L.HipValueError(f'no k-means workspace for B={B} H={H} D={D} M={M}')
         ws = self._ws.get(str(device))
@@ -115,9 +115,10 @@ class BoundaryMemory:
         iters = ITERS_INIT if cold else ITERS_UPDATE
         rep = torch.empty(H, M, dtype=torch.long, device=dev)
         valid = torch.empty(H, M, dtype=torch.bool, device=dev)
-        ws = self._workspace(B, H, D, M, iters, dev)
+        fp32_keys = int(keys.dtype == torch.float32)
+        ws = self._workspace(B, H, D, M, iters, fp32_keys, dev)
         with torch.cuda.device(dev):
-            L.check(L.lib().or_memory_select(keys.data_ptr(), int(keys.dtype == torch.float32), L.ptr(rows),
+            L.check(L.lib().or_memory_select(keys.data_ptr(), fp32_keys, L.ptr(rows),
                                              keys.stride(0), B, H, D, M, c.data_ptr(),
                                              init.data_ptr() if cold else None, iters, rep.data_ptr(),
                                              valid.data_ptr(), ws.data_ptr(), ws.numel(), L.stream_handle(dev)),

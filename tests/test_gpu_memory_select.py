@@ -5,6 +5,7 @@ clusters (more groups than clusters would leave ties)."""
 import pytest
 import torch
 
+from onereel_amd import _lib as L
 from onereel_amd.memory import BoundaryMemory
 
 pytestmark = [pytest.mark.gpu, pytest.mark.skipif(not torch.cuda.is_available(), reason='needs the GPU')]
@@ -44,3 +45,23 @@ def test_select_passes(B, H, D, M, dtype):
             assert torch.equal(group[chosen], torch.arange(M))
             for i in range(M):              # nearest up to the rounding of |x|^2 - 2 x.c + |c|^2 near 1
                 assert d[chosen[i]] <= d[group == i].min() + 1e-6
+
+
+@pytest.mark.parametrize('B,H,D,M,dtype', [(777, 3, 128, 40, torch.bfloat16), (33, 1, 64, 7, torch.bfloat16),
+                                           (777, 3, 128, 40, torch.float32)])
+def test_workspace_of_each_key_type(B, H, D, M, dtype):
+    """a call within exactly the bytes that its key type needs: nothing past them is written"""
+    print(f'select workspace B={B} H={H} D={D} M={M} {dtype}', flush=True)
+    x = torch.randn(B, H, D, generator=torch.Generator().manual_seed(B)).to(dtype).to(DEV)
+    mem, fp32 = BoundaryMemory(M), int(dtype == torch.float32)
+    rep, valid = mem.select('a', x)
+    n = int(L.lib().or_memory_select_workspace_bytes(B, H, D, M, 50, fp32))
+    ws = torch.full((n + 4096,), 0x5a, dtype=torch.uint8, device=DEV)
+    c = torch.empty(H, M, D, device=DEV)
+    init = torch.linspace(0, B - 1, M).round().to(torch.int32).to(DEV)
+    got, ok = torch.empty_like(rep), torch.empty_like(valid)
+    L.check(L.lib().or_memory_select(x.data_ptr(), fp32, None, x.stride(0), B, H, D, M, c.data_ptr(), init.data_ptr(),
+                                     50, got.data_ptr(), ok.data_ptr(), ws.data_ptr(), n, L.stream_handle(x.device)),
+            'or_memory_select')
+    assert torch.equal(got, rep) and torch.equal(ok, valid) and torch.equal(c, mem.centroids['a'])
+    assert bool((ws[n:] == 0x5a).all())

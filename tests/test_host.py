@@ -563,3 +563,17 @@ def test_frame_select_hands_over_candidates_in_host_memory(monkeypatch, default)
     feats = torch.randn(7, 16, device='cpu')
     with torch.device(default):
         assert fm.select(feats) == fm.candidate_frames()[:3] == [0, 1, 2]
+
+
+def test_memory_workspace_of_bf16_keys_holds_no_normalised_keys():
+    size, size_of = L.lib().or_memory_select_workspace_size, L.lib().or_memory_select_workspace_bytes
+    for B, H, D, M, iters in ((12720, 16, 128, 128, 2), (5, 1, 64, 3, 50)):
+        x = (H * B * D * 4 + 255) // 256 * 256
+        assert size_of(B, H, D, M, iters, 1) == size(B, H, D, M, iters) == size_of(B, H, D, M, iters, 0) + x
+    assert size_of(5, 1, 96, 3, 2, 0) == size(5, 1, 96, 3, 2) == -1
+    a = 0x10000
+    for fp32 in (0, 1):   # one byte short of either
+        n = size_of(100, 2, 128, 8, 2, fp32)
+        with pytest.raises(L.HipPathError, match=f'workspace of {n} bytes'):
+            L.check(L.lib().or_memory_select(a, fp32, a, 256, 100, 2, 128, 8, a, None, 2, a, a, a, n - 1, None),
+                    'or_memory_select')
