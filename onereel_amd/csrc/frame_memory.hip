@@ -8,11 +8,14 @@
 //
 // - frame_pool_kernel: rows are frame-major (frame of row r = (row0 + r) / T, as the one-GPU processors build
 //   them), so a frame's rows are contiguous. A block per (frame, 128 columns) adds them in row order:
-//   deterministic, unlike an atomic index_add_. Per lane, 2 consecutive columns in fp32.
+//   deterministic, unlike an atomic index_add_. Per lane, 2 consecutive columns in fp32. With many short frames
+//   frame_pool_wave_kernel, a wavefront per (frame, 512 columns), in the same order: the same bits.
 // - frame_select_kernel: the whole selection in one workgroup of 1024 threads, centres in LDS (k * C floats); no
 //   host round trip per iteration. Ties are broken towards the lower index, as torch.argmax does. A pass stops when
 //   the new centres equal the old ones exactly (torch.equal).
 #include <math.h>
+
+#include <algorithm>
 
 #include "common.h"
 
@@ -92,6 +95,57 @@ __global__ __launch_bounds__(kPoolThreads) void frame_pool_kernel(PoolArgs g) {
     sp[1] += a1;
     if (col == 0) g.counts[f] += (float)n;
   }
+}
+
+// The same sums, a wavefront per (frame, 512 columns): eight columns per lane, four rows in flight, no LDS and no barrier.
+// Where its wavefronts fill the chip by themselves, what a block of frame_pool_kernel costs beside the rows (a stage of 64
+// rows however few there are, the barriers) is what counts: 5000 frames of one row of 1024 columns 46 -> 7 us, 240 frames
+// of 48 rows x 3072 columns 16.6 -> 12.5.
+__global__ __launch_bounds__(kPoolThreads) void frame_pool_wave_kernel(PoolArgs g) {
+  const int lane = threadIdx.x & 63;
+  const int cb = blockIdx.x * (kPoolThreads / 64) + (threadIdx.x >> 6);   // 512-column block
+  const int f = blockIdx.y, col = cb * 512 + 8 * lane;
+  int64_t r0 = (int64_t)f * g.T - g.row0, r1 = r0 + g.T;
+  r0 = r0 < 0 ? 0 : r0;
+  r1 = r1 > g.n_rows ? g.n_rows : r1;
+  if (r1 <= r0 || col >= g.C) return;
+  float acc[8] = {};
+  auto add = [&](const u32x4& v) {
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      acc[2 * p] += bf2f((uint16_t)(v[p] & 0xffffu));
+      acc[2 * p + 1] += bf2f((uint16_t)(v[p] >> 16));
+    }
+  };
+  const uint16_t* p = g.hs + r0 * g.row_stride + col;
+  int n = (int)(r1 - r0);
+  for (; n >= 4; n -= 4, p += 4 * g.row_stride) {
+    u32x4 v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v[u] = *(const u32x4*)(p + u * g.row_stride);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) add(v[u]);
+  }
+  for (; n > 0; --n, p += g.row_stride) add(*(const u32x4*)p);
+  float* sp = g.sums + (int64_t)f * g.C + col;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) sp[e] += acc[e];
+  if (col == 0) g.counts[f] += (float)(r1 - r0);
+}
+
+// Which of the two pools a call: w wavefronts of 512 columns. Staged / direct, us: up to 32 rows a frame the direct kernel
+// from 400 wavefronts on (20 000 frames x 16 rows x 64 columns 36 / 19, 100 x 24 x 3072 5.7 / 4.4; 1000 x 24 x 64, 125
+// wavefronts, 3.7 / 5.8), up to 48 from 1500 on (20 000 x 48 x 64 46 / 39; 5000 x 48 x 128, 1250, 12.7 / 16). Past that only
+// with whole wavefronts of columns (5000 x 64 x 128: 16.5 / 19.4) and from 700 on, where a stage or two are less than full
+// (200 x 64 x 2048 12.0 / 11.0, 240 x 192 x 2048 29.6 / 27.4; 150 x 64 x 2048, 600 wavefronts, 9.7 / 10.1; 400 x 128 x 3072,
+// 2400 wavefronts, 51 / 59), or while eight wavefronts per CU hold the whole call (240 x 1590 x 3072 404 / 384, 400 x 1590 x
+// 2048 446 / 422; 240 x 1590 x 2048, 960 wavefronts, 269 / 302; 400 x 1590 x 3072, 2400 wavefronts, 670 / 761).
+static bool pool_by_wave(int64_t frames, int C, int T) {
+  const int64_t w = frames * C / 512;
+  if (T <= 32) return w >= 400;
+  if (T <= 48 && w >= 1500) return true;
+  if (C < 512 || w < 700) return false;
+  return T <= 96 || (w <= 2048 && (T < 200 || w >= 1200));
 }
 
 // sum over the 64 lanes, the same in every lane: the tree of a butterfly with partners 32, 16, 8, 4, 2 and 1 lanes away,
@@ -399,8 +453,12 @@ extern "C" int or_frame_pool(const void* hs, int64_t n_rows, int32_t C, int64_t 
                     n_frames);
   if (((uintptr_t)hs & 15u) || row_stride % 8) return fail_arg("or_frame_pool: hs must be 16-byte aligned rows");
   PoolArgs g{(const uint16_t*)hs, n_rows, row_stride, row0, C, T, n_frames, sums, counts};
-  hipLaunchKernelGGL(frame_pool_kernel, dim3((unsigned)((C + 127) / 128), (unsigned)n_frames), dim3(kPoolThreads), 0,
-                     (hipStream_t)stream, g);
+  if (pool_by_wave(std::min<int64_t>(n_frames, n_rows / T + 1), C, T))
+    hipLaunchKernelGGL(frame_pool_wave_kernel, dim3((unsigned)((C + 2047) / 2048), (unsigned)n_frames), dim3(kPoolThreads),
+                       0, (hipStream_t)stream, g);
+  else
+    hipLaunchKernelGGL(frame_pool_kernel, dim3((unsigned)((C + 127) / 128), (unsigned)n_frames), dim3(kPoolThreads), 0,
+                       (hipStream_t)stream, g);
   return check_hip(hipGetLastError(), "frame_pool_kernel launch");
 }
 
