@@ -6,7 +6,9 @@ point raises.
 """
 from __future__ import annotations
 
+import array
 import ctypes
+import itertools
 import os
 from pathlib import Path
 
@@ -203,13 +205,18 @@ def device_ints(lists, device):
     values (a copy from pageable memory would cost each list about 10 us of the host's time). The launches are queued on
     the device's current stream and not waited for: for a call that reads the values on that stream, not for tensors
     that are handed out"""
-    flat = [int(x) for values in lists for x in values]
-    if device is None or torch.device(device).type != 'cuda' or not flat or min(flat) < -2 ** 31 or max(flat) >= 2 ** 31:
+    flat = None
+    if device is not None and torch.device(device).type == 'cuda':
+        try:
+            flat = array.array('i', itertools.chain(*lists))
+        except (OverflowError, TypeError):
+            pass            # values that are no 32-bit integers: torch's conversions and its errors
+    if not flat:
         return [torch.tensor(list(values), dtype=torch.int32, device=device) for values in lists]
     out = torch.empty(len(flat), dtype=torch.int32, device=device)
     with torch.cuda.device(out.device):
-        check(lib().or_index_fill((ctypes.c_int32 * len(flat))(*flat), len(flat), out.data_ptr(),
-                                  stream_handle(out.device)), 'or_index_fill')
+        check(lib().or_index_fill(flat.buffer_info()[0], len(flat), out.data_ptr(), stream_handle(out.device)),
+              'or_index_fill')
     return list(out.split([len(values) for values in lists]))
 
 

@@ -17,8 +17,9 @@ def test_device_ints(sizes):
         assert got.dtype == torch.int32 and got.cpu().tolist() == want
 
 
+# up to 112 sequences, and long ones past them, in or_concat's launches; many short ones by torch
 @pytest.mark.parametrize('n,H,D,most', [(1, 1, 64, 5), (3, 24, 128, 400), (112, 2, 64, 40), (113, 2, 128, 40),
-                                        (250, 1, 64, 9)])
+                                        (250, 1, 64, 9), (113, 16, 128, 300), (250, 16, 128, 200)])
 def test_concat(n, H, D, most):
     print(f'concat n={n} H={H} D={D}', flush=True)
     g = torch.Generator(device=DEV).manual_seed(n)
@@ -30,7 +31,7 @@ def test_concat(n, H, D, most):
         assert torch.equal(got, torch.cat(parts))
     assert cu_q.cpu().tolist() == A._offsets(nq) and cu_k.cpu().tolist() == A._offsets([k.shape[0] for _, k, _ in seg])
     assert (max_q, max_k) == (max(nq), max(k.shape[0] for _, k, _ in seg))
-    # rows that are not contiguous are concatenated by torch: the same tensors
+    # what or_concat does not take is concatenated by torch: the same tensors
     wide = [(torch.cat([q, q], 2)[..., :D], k, v) for q, k, v in seg]
     assert torch.equal(A._concat(wide)[0][0], q) and torch.equal(A._concat(wide)[0][3], cu_q)
 
@@ -49,3 +50,14 @@ def test_cu_seqlens_are_there_on_return():
         got = cu.cpu()
     torch.cuda.synchronize()
     assert got.tolist() == want
+
+
+def test_device_ints_takes_what_torch_takes():
+    """values that are no 32-bit integers convert or fail as torch's do; empty lists, numpy integers and tensors"""
+    import numpy as np
+    for lists in ([[1.9, -2.9]], [[True, 3]], [[np.int64(7), torch.tensor(5)]], [[], []], [[], [4], []], [[2 ** 31 - 1, -2 ** 31]]):
+        for got, values in zip(L.device_ints(lists, DEV), lists):
+            assert torch.equal(got.cpu(), torch.tensor(list(values), dtype=torch.int32)) and got.is_cuda
+    for bad in (2 ** 31, -2 ** 31 - 1):
+        with pytest.raises((RuntimeError, OverflowError)):
+            L.device_ints([[bad]], DEV)
