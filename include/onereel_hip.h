@@ -273,8 +273,12 @@ int64_t or_varlen_workspace_size(int32_t n_seg, int32_t sum_q, int32_t H, int32_
 /* Replaces attention.varlen / flash_attn_varlen_func (src/onereel/attention.py:39-43), varlen_lse (:46-53) and
  * overlapping_ranges' FA3 call with seqused_k (:78-83): non-causal softmax(q k^T * scale) v per segment, bf16 in and
  * out, fp32 accumulation. Two launches: a tile planner and the attention kernel (64 queries per wavefront at
- * D = 128, 32 at D = 64), and a third that merges key-split items when a call may have them; one launch when D = 128,
- * max_k is at most 256 and none of seg_q_src, q_rope, k_len_head, v_tok and k_tok is set. */
+ * D = 128, 32 at D = 64), and a third that merges key-split items when a call may have them. Calls of at most 256
+ * segments take one launch in two forms, which leave the workspace as it is: at D = 128 when max_k is 1 to 256 and none
+ * of seg_q_src, q_rope, k_len_head, v_tok and k_tok is set (keys and values of a segment-head in LDS); at D = 64 when
+ * (sum_q + 127 n_seg) / 128 * H items are resident on the device at once. A segment's results have the same bits in
+ * every form, but where the planner splits its items by keys (D = 128, calls of fewer than four rounds of items), or,
+ * between the forms of D = 128, where a row's probabilities sum to more than 2^20 of the running maximum. */
 int or_varlen_fwd(const or_varlen_args* args, void* stream);
 
 /* Bytes of the device array that or_varlen_fwd_noalloc uses in place of a caller workspace (one per GPU). */

@@ -554,10 +554,11 @@ __device__ __forceinline__ float pair_sum(float x) {
 
 // ------------------------------------------------------------------------------------------------------------------
 // Ring kernel with 32 queries per wavefront (attn4_kernel, run for head_dim 64): software-pipelined over blocks of
-// 32 keys. K and V blocks stream through two rings of four LDS slots each, filled by buffer loads straight into LDS (LDS DMA) three iterations ahead; rows past a
-// segment's end read as zeros. Iteration j of a wavefront runs the softmax of block j on the VALU while the MFMA unit
-// computes S of block j + 1 (QK^T) and O += V P^T of block j - 1, so the exponentials overlap the matrix work inside
-// one wavefront as well as across the wavefronts that share a SIMD. At head_dim 64 the vector work (55 instructions, 16 of
+// 32 keys. K and V blocks stream through two rings of four LDS slots each, filled by buffer loads straight into LDS
+// (LDS DMA) three iterations ahead; rows past a segment's end read as zeros. Iteration j of a wavefront runs the softmax
+// of block j on the VALU while the MFMA unit computes S of block j + 1 (QK^T) and O += V P^T of block j - 1, so the
+// exponentials overlap the matrix work inside one wavefront as well as across the wavefronts that share a SIMD. At
+// head_dim 64 the vector work (55 instructions, 16 of
 // them exponentials, per 8 MFMAs) is longer than the matrix work, and a wavefront also waits for its LDS reads and its
 // block's barrier: a third wavefront per SIMD (145 registers, 33 KB of LDS per block; a fourth would spill) fills those
 // waits: 4 x 8192 x 8192 x 16 heads 929 -> 990 TFLOP/s, 2 x 3001 x 3001 x 16 (768 blocks in one round instead of 1.5)

@@ -319,9 +319,10 @@ __global__ __launch_bounds__(kThreads) void index_fill_kernel(FillArgs g, int n,
 }
 
 // The rows of up to kCatSegs q, k and v tensors end to end, and the two offset arrays of a varlen call, in one launch
-// (three concatenations and two copies of offsets before it: 44 us of GPU time for 12 sequences of 3111 query and 3638
-// key rows x 16 heads x 128, now 15). HBM-bound (every byte read and written once): a block writes 16-byte chunks of one of the
-// three results, each thread finding its chunk's sequence among the offsets in LDS; eight chunks in flight per thread.
+// (three concatenations and two copies of offsets before it: 44 us of GPU time for 12 sequences of together 3111 query and
+// 3638 key rows x 16 heads x 128, now 15). HBM-bound (every byte read and written once): a block writes 16-byte chunks of
+// one of the three results, each thread finding its chunk's sequence among the offsets in LDS; eight chunks in flight per
+// thread.
 constexpr int kCatSegs = 112;
 constexpr int kCatFly = 8;
 struct CatArgs {
