@@ -8,6 +8,7 @@ import torch
 
 from helpers import assert_close, rand_bf16
 from onereel_amd import scene
+from onereel_amd.layout import SceneLayout
 from oracle import attention as OA
 
 pytestmark = [pytest.mark.gpu, pytest.mark.skipif(not torch.cuda.is_available(), reason='needs the GPU')]
@@ -102,3 +103,19 @@ def test_short_keys_running_max_moves(n_keys):
     first, last = (s[:, :, block == b].amax(-1) for b in (0, nb - 1))
     assert bool((last - first > 20).any()) and bool(((last - first > 0.5) & (last - first < 4)).any())
     _check(o.cpu(), lse.cpu(), q, k, v, [n], [n_keys])
+
+
+def test_small_scopes_fused_and_packed_agree(monkeypatch):
+    """a scene layer whose scopes have at most 256 keys: the packed flow's call takes the short form, the fused one's (queries
+    by source row) the ring kernel, here without key splits: the same bits"""
+    lengths, T, counts, H, D = [2, 1, 2], 50, [20, 33, 7], 6, 128
+    S, Le = sum(lengths) * T, sum(counts)
+    q, k, v = (rand_bf16((S, H, D), 31 + i).to(DEV) for i in range(3))
+    eq, ek, ev = (rand_bf16((Le, H, D), 41 + i).to(DEV) for i in range(3))
+    cos, sin = (x.to(DEV) for x in OA.rope_table_3d(8, 5, 10, D))
+    plan = scene.ScopePlan(SceneLayout(lengths, halo=0, extra={0: [3], 1: [0, 4], 2: []}), T, counts, Le, True, None, True,
+                           True, torch.device(DEV))
+    assert 128 < plan.max_k <= 256
+    monkeypatch.setenv('ONEREEL_ATTN_MAX_BLOCKS', '1')
+    a, b = (scene.scene_attention(plan, q, k, v, eq, ek, ev, cos, sin, mode='raw', fused=fused) for fused in (True, False))
+    assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
